@@ -42,6 +42,7 @@ struct awp_batch {
     bool split;                  // two-stage scheme (else fused)
     bool can_fuse;               // every run holds the fused scheme's two buffers
     bool persist;                // persistent grids (else one block per tile)
+    bool claims;                 // persistent two-stage blocks claim their tiles (AWP_CLAIM is not 0)
     bool o32;                    // 32-bit byte offsets reach every run's arrays
     Launch l;                    // tile_y and prefetch depth / z unroll (unroll) of the batch
     std::vector<int> nchunk;     // fused scheme: z chunks per run
@@ -196,7 +197,7 @@ static hipError_t launch_kernels(awp_batch *b, int par)
     const int n = (int)b->runs.size();
     if (b->split)
         return launch_step_split_batch(b->mixed, b->l, b->o32, b->d_sjobs, n, b->total, b->fs_total,
-                                       b->grid_v, b->grid_s, b->persist && b->l.claim != 0 ? b->d_claim : nullptr,
+                                       b->grid_v, b->grid_s, b->persist && b->claims ? b->d_claim : nullptr,
                                        b->stream);
     return launch_step_fused_batch(b->mixed, b->l, b->d_jobs, n, b->total, b->grid, par, b->d_claim, b->stream);
 }
@@ -291,7 +292,11 @@ extern "C" int awp_batch_create(awp_batch **out, awp_ctx *const *runs, int nruns
     const char *bs = getenv("AWP_BATCH_SCHEME");
     if (bs && !strcmp(bs, "fused") && b->can_fuse) b->split = false;
     if (bs && !strcmp(bs, "split")) b->split = true;
-    b->persist = true;
+    // two-stage: one block per tile (see choose_launch's tile claim); the
+    // fused kernel's blocks claim
+    const char *ce = getenv("AWP_CLAIM");
+    b->persist = !b->split || (ce && !strcmp(ce, "2"));
+    b->claims = !(ce && !strcmp(ce, "0"));
     b->o32 = true;
     for (int r = 0; r < nruns; ++r) b->o32 = b->o32 && runs[r]->l.o32;
     b->l = runs[0]->l;
@@ -299,6 +304,7 @@ extern "C" int awp_batch_create(awp_batch **out, awp_ctx *const *runs, int nruns
         // two-stage kernels: {64, 128} x {1, 2, 4, 8} tiles, z unroll 1 or 2;
         // blocks of more than 512 threads (64 x 16, 128 x 8) in the
         // byte-offset stress form without z unroll
+        if (runs[0]->fused) b->l.tile_y = 4;   // a fused run's launch shape is no guide
         if (b->l.unroll != 2) b->l.unroll = 1;
         if (b->l.tile_xw != 2) b->l.tile_xw = 1;
         const bool tall_ok = b->o32 && b->l.o32_s && b->l.unroll == 1;
@@ -315,7 +321,16 @@ extern "C" int awp_batch_create(awp_batch **out, awp_ctx *const *runs, int nruns
         b->l.tile_xw = 1;
     }
     b->nchunk.assign(nruns, 1);
-    b->kc_split = SPLIT_KC;
+    // the chain of a wave's levels is hidden by every run's waves together
+    {
+        long long rows = 0;
+        int nz = 0;
+        for (int r = 0; r < nruns; ++r) {
+            rows += row_segments(runs[r]->g);
+            nz = std::max(nz, runs[r]->g.nz);
+        }
+        b->kc_split = split_kc(rows, nz);
+    }
     b->d_jobs = nullptr;
     b->d_sjobs = nullptr;
     b->d_aux = nullptr;
@@ -453,22 +468,24 @@ extern "C" int awp_batch_tune(awp_batch *b, int reps)
         bool split, persist;
         int ty, pf, nchunk;   // nchunk: z chunks per run (fused), chunk length in levels (two-stage)
         int xw;      // two-stage: waves per tile row
-        int sform;   // two-stage stress kernel: 0 = 64-bit offsets, blocks as registers allow;
-                     // 1 = 32-bit offsets, 2 blocks per CU
+        int sform;   // two-stage stress kernel: 0 = 64-bit offsets, 1 = 32-bit offsets, 2 blocks per
+                     // CU; 2 = 32-bit offsets (0 and 2: blocks as registers allow)
         bool patch;  // two-stage: the runs' tile patches (else rows of tiles)
     };
     std::vector<Cand> cands;
+    // two-stage, one block per tile, chunk lengths about the default's
+    for (int kc : {b->kc_split * 2 / 3, b->kc_split, b->kc_split * 3 / 2})
+        for (bool pt : {true, false}) cands.push_back({true, false, 4, 1, std::max(4, kc), 1, b->o32 ? 2 : 0, pt});
     for (bool ps : {true, false}) {
-        // two-stage: tile rows x z unroll x z chunk length (levels) x stress
-        // kernel form x tile order
+        // two-stage: tile rows x z chunk length (levels) x stress kernel form
+        // x tile order
         for (int ty : {4, 8})
-            for (int un : {1, 2})
-                for (int kc : {SPLIT_KC, 2 * SPLIT_KC})
-                    for (int sf : {0, 1})
-                        for (bool pt : {true, false}) cands.push_back({true, ps, ty, un, kc, 1, sf, pt});
+            for (int kc : {25, 50})
+                for (int sf : {0, 1})
+                    for (bool pt : {true, false}) cands.push_back({true, ps, ty, 1, kc, 1, sf, pt});
         // 128 x 4 tiles; 64 x 16 and 128 x 8 tiles (1024-thread blocks:
         // byte-offset stress form, no z unroll)
-        for (int kc : {SPLIT_KC, 2 * SPLIT_KC})
+        for (int kc : {25, 50})
             for (bool pt : {true, false}) {
                 for (int sf : {0, 1}) cands.push_back({true, ps, 4, 1, kc, 2, sf, pt});
                 if (b->o32) {
@@ -486,7 +503,7 @@ extern "C" int awp_batch_tune(awp_batch *b, int reps)
     }
     const int spw0 = b->l.spw, sph0 = b->l.sph;
     auto apply_form = [b, spw0, sph0](int sf, bool patch) {
-        b->l.o32_s = sf == 1;
+        b->l.o32_s = sf != 0;
         b->l.bpc_s = sf == 1 ? 2 : 0;
         b->l.spw = patch ? spw0 : 0;
         b->l.sph = patch ? sph0 : 0;

@@ -126,6 +126,17 @@ static bool want_fused(const Geo &g, int storage)
     return storage == AWP_STORAGE_FP32;
 }
 
+// Whether a run that holds both buffers starts on the fused step: always
+// under AWP_SCHEME=fused, else from 200M points on.  FP32, two-stage against
+// fused on the same buffers: 200x200x100 0.20 against 0.23 ms per step,
+// 517x389x149 1.24 against 1.29, 800x600x200 3.60 against 3.74, 1500x1000x300
+// 17.1 against 16.8.
+static bool start_fused(const Geo &g)
+{
+    const char *scheme = getenv("AWP_SCHEME");
+    return (scheme && !strcmp(scheme, "fused")) || (long long)g.nx * g.ny * g.nz >= 200000000ll;
+}
+
 // z chunks of `nchunk` requested: the top chunk keeps >= 3 levels (the
 // block reaching k = nz writes the free-surface stress images from the two
 // levels below it)
@@ -156,7 +167,15 @@ static void set_chunks(Launch &l, const Geo &g, int nchunk, bool fused)
 static Launch choose_launch(const Geo &g, bool fused, bool mixed, int device)
 {
     Launch l;
-    l.tile_y = 8;
+    // two-stage: 64 x 4 tiles, 64 x 2 where the chunks are short (split_kc).
+    // Low tiles share no less in the caches than tall ones (the L2 serves
+    // both) and small blocks fill the wave slots evenly: one block per tile,
+    // ms per step with 2 / 4 / 8 rows, FP32 and mixed: 131x97x53 (4 levels)
+    // 0.060 / 0.062 / 0.066 and 0.059 / 0.061 / 0.064; 400x300x150 (17) 0.749
+    // / 0.749 / 0.771 and 0.636 / 0.639 / 0.659; 1410x88x77 (13) 0.427 /
+    // 0.404 / 0.394; 800x600x200 (25) 3.60 / 3.62 / 3.65 and 2.99 / 2.99 /
+    // 3.02; 1500x1000x300 17.08 / 17.17 / 17.25 and 14.21 / 14.20 / 14.28
+    l.tile_y = split_kc(row_segments(g), g.nz) > 8 ? 4 : 2;
     l.tile_xw = 1;
     l.unroll = 1;
     const char *un = getenv("AWP_UNROLL");
@@ -174,20 +193,21 @@ static Launch choose_launch(const Geo &g, bool fused, bool mixed, int device)
                atoi(ty) == 16))
         l.tile_y = atoi(ty);
     if (fused && l.tile_y != 4 && l.tile_y != 7 && l.tile_y != 11) l.tile_y = 8;
-    if (!fused && l.tile_y == 11) l.tile_y = 8;
-    if (!fused && l.tile_y == 7) l.tile_y = 8;
+    if (!fused && (l.tile_y == 7 || l.tile_y == 11)) l.tile_y = 8;
     // tile patches of the fused step (AWP_PATCH=<w>x<h> overrides): 4 x 4
     // tiles of 64 x 8 points (1500x1000x300 FP32, 4 z chunks: 17.21 ms per
     // step against 17.62 for 2 x 16 and 17.75 for 3 x 8)
     l.pw = 4;
     l.ph = 4;
     // tile claim (AWP_CLAIM=0 never, 1 when the launch has at least four
-    // tiles per persistent block -- the default --, 2 always; AWP_XROT=0..7
-    // rotates the XCD ranges): persistent blocks that claim tiles per XCD.
-    // 1500x1000x300: fused 16.81-16.92 ms per step against 17.11-17.20 with
-    // one block per tile (same run); 200x200x100 (400 two-stage tiles) one
-    // block per tile is faster
-    l.claim = 1;
+    // tiles per persistent block, 2 always; AWP_XROT=0..7 rotates the XCD
+    // ranges): persistent blocks that claim tiles per XCD.  The fused step's
+    // default (1500x1000x300: 16.81-16.92 ms per step against 17.11-17.20
+    // with one block per tile, same run); the two-stage kernels run one block
+    // per tile, whose dispatch costs less than a claim per short tile
+    // (400x300x150, 64 x 2 tiles of 17 levels: 0.749 ms per step against
+    // 0.923 claimed)
+    l.claim = fused ? 1 : 0;
     l.xrot = 0;
     const char *ce = getenv("AWP_CLAIM");
     if (ce && (!strcmp(ce, "0") || !strcmp(ce, "1") || !strcmp(ce, "2"))) l.claim = ce[0] - '0';
@@ -273,9 +293,11 @@ static Launch choose_launch(const Geo &g, bool fused, bool mixed, int device)
         // 3 chunks ran 16.21-16.23 ms per step on two boxes; 4 chunks
         // 16.34 on one and 17.71 on the other, 2 chunks 17.92 (each chunk
         // recomputes 4 velocity levels)
-        nchunk = std::max(1, (g.nz + 50) / 100);
+        // Grids of few tile columns take more chunks, four tiles per CU
+        // (517x389x149, 324 columns: one chunk 1.66 ms per step, two 1.37,
+        // three 1.29, six 1.29)
+        nchunk = std::max<long long>(std::max(1, (g.nz + 50) / 100), (1024 + bxy / 2) / bxy);
         nchunk = std::min(nchunk, std::max(1, g.nz / 16));
-        (void)bxy;
     } else if (fused) {
         // 64 x 8, 64 x 7, 64 x 4 tiles: an even number of chunks of about
         // 75 levels (1500x1000x300, 64 x 8: 17.2-17.7 ms per step with 2 or
@@ -283,12 +305,7 @@ static Launch choose_launch(const Geo &g, bool fused, bool mixed, int device)
         nchunk = 2 * std::max(1, (g.nz + 75) / 150);
         nchunk = std::min(nchunk, std::max(1, g.nz / 16));
     } else {
-        // z chunks of about SPLIT_KC levels: with the tile patches, the
-        // tiles an XCD holds at once then span few levels and share their
-        // halo lines in L2 (1500x1000x300: chunks of 150 levels 18.64 ms
-        // per step FP32, 17.46 mixed; of 25 levels 18.29 and 16.25; of 12,
-        // 18.57 and 16.37 -- the z queues' start-up loads take over)
-        nchunk = split_nchunk(g.nz, SPLIT_KC);
+        nchunk = split_nchunk(g.nz, split_kc(row_segments(g), g.nz));
     }
     const char *kc_env = getenv("AWP_KC");
     if (kc_env && atoi(kc_env) >= 3) nchunk = std::max(1, (g.nz + atoi(kc_env) - 1) / atoi(kc_env));
@@ -322,8 +339,8 @@ extern "C" int awp_create(awp_ctx **out, const awp_in3d *p, int device, int stor
     ctx->device = device;
     ctx->storage = storage;
     ctx->g = make_geo(p->nx, p->ny, p->nz);
-    ctx->fused = want_fused(ctx->g, storage);
-    ctx->two_bufs = ctx->fused;
+    ctx->two_bufs = want_fused(ctx->g, storage);
+    ctx->fused = ctx->two_bufs && start_fused(ctx->g);
     ctx->l = choose_launch(ctx->g, ctx->fused, storage == AWP_STORAGE_MIXED, device);
     ctx->vol = nullptr;
     ctx->prof = nullptr;
@@ -1006,9 +1023,8 @@ extern "C" int awp_tune(awp_ctx *ctx, int reps)
     HIPTRY(ctx, hipSetDevice(ctx->device));
     int rc = ensure_events(ctx, 2);
     if (rc) return rc;
-    // candidates: the two-stage step with its defaults, and on grids of
-    // fewer tiles than the GPU holds blocks (200x200x100: 400 tiles) with
-    // shorter z chunks and 64 x 4 tiles for more of them; with both buffers,
+    // candidates: the two-stage step with its defaults, with shorter and
+    // longer z chunks and on taller tiles; with both buffers,
     // the fused step on 64 x 11 tiles (FP32; z chunks of about 100, 75, 60
     // levels x tile patches 4x4, 2x2, 8x2, and larger patches) and 64 x 8
     // tiles, or on 64 x 7 tiles (mixed).  The fastest is kept.
@@ -1019,11 +1035,11 @@ extern "C" int awp_tune(awp_ctx *ctx, int reps)
     std::vector<Cand> cands;
     cands.push_back({false, 0, 0, 0, 0});
     {
-        const long long tiles = (long long)((ctx->g.nx + TX - 1) / TX) * ((ctx->g.ny + 7) / 8) *
-                                split_nchunk(ctx->g.nz, SPLIT_KC);
-        if (tiles < 4096)
-            for (int ty : {8, 4})
-                for (int kc : {12, 8}) cands.push_back({false, ty, kc, 0, 0});
+        const int kc = split_kc(row_segments(ctx->g), ctx->g.nz);
+        cands.push_back({false, 4, std::max(4, kc * 2 / 3), 0, 0});
+        cands.push_back({false, 4, kc * 3 / 2, 0, 0});
+        cands.push_back({false, kc > 8 ? 2 : 4, kc, 0, 0});
+        cands.push_back({false, 8, 25, 0, 0});
     }
     if (ctx->two_bufs) {
         if (!ctx->mixed()) {

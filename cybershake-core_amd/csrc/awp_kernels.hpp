@@ -389,8 +389,30 @@ struct Cursor32 {
     __device__ __forceinline__ void up() { o += sz; }
 };
 
-// z chunks of the two-stage kernels: about `kc` levels each
-constexpr int SPLIT_KC = 25;
+// z chunk length of the two-stage kernels for `rows` row segments of 64
+// points a level and nz levels.  A wave marches its chunk level by level, 2.9
+// us each on an idle GPU (load, compute, store), so a grid that cannot fill
+// the GPU's 4096 wave slots (4 per SIMD) is bound by that chain and takes
+// short chunks: about three waves per slot, 4 to 17 levels each (below 4 the
+// z queues' start-up loads cost more than the shorter chain saves).  From
+// twelve waves per slot on the chain is hidden and 25-level chunks, with
+// fewer start-up loads, win.  Milliseconds per step, 64 x 2 tiles, one block
+// per tile, FP32 / mixed: 48x40x32 with 4 / 12 levels 0.032 / 0.044 and
+// 0.037 / 0.049; 131x97x53 with 4 / 25 levels 0.060 / 0.092 and 0.059 /
+// 0.124; 300x250x80 with 8 / 25 0.261 / 0.275 and 0.231 / 0.257; 400x300x150
+// with 17 / 25 0.749 / 0.765 and 0.636 / 0.668; 800x600x200 with 17 / 25 3.71
+// / 3.60 and 3.07 / 2.99; 1500x1000x300 with 12 / 17 / 25 / 50 17.25 / 17.23 /
+// 17.08 / 17.39 and 14.37 / 14.32 / 14.21 / 14.32.
+static inline int split_kc(long long rows, int nz)
+{
+    const long long waves = rows * nz;   // row segments over the whole volume
+    if (waves >= 25ll * 12 * 4096) return 25;
+    const long long kc = waves / (3 * 4096);
+    return kc < 4 ? 4 : kc > 17 ? 17 : (int)kc;
+}
+// row segments of 64 points per level of a grid
+static inline long long row_segments(const Geo &g) { return (long long)((g.nx + 63) / 64) * g.ny; }
+// z chunks of about `kc` levels each
 static inline int split_nchunk(int nz, int kc)
 {
     const int n = (nz + kc / 2) / kc;
