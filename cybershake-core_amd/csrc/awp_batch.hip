@@ -53,7 +53,7 @@ struct awp_batch {
     AuxJob *d_aux;
     int *d_counter;
     unsigned long long *d_claim;   // the fused kernel's tile claim counters (CLAIM_WORDS)
-    int total, fs_total, max_kept;
+    int total, max_kept;
     int grid, grid_v, grid_s;    // persistent blocks: fused kernel; velocity, stress kernels
     hipGraphExec_t graph;
     bool graph_ok;
@@ -122,7 +122,7 @@ static int upload_tables(awp_batch *b)
     std::vector<FJob> fj(n);
     std::vector<SJob> sj(n);
     std::vector<AuxJob> aj(n);
-    int tile0 = 0, fs0 = 0;
+    int tile0 = 0;
     b->max_kept = 0;
     for (int r = 0; r < n; ++r) {
         awp_ctx *c = b->runs[r];
@@ -131,9 +131,8 @@ static int upload_tables(awp_batch *b)
         AuxJob &x = aj[r];
         if (b->split) {
             SJob &q = sj[r];
-            q = split_job(c->g, c->view(c->cur), c->c, l, tile0, fs0);
+            q = split_job(c->g, c->view(c->cur), c->c, l, tile0);
             tile0 += split_tiles(q);
-            fs0 += split_fs_blocks(q);
             x.s[0] = x.s[1] = q.s;
         } else {
             FJob &f = fj[r];
@@ -170,7 +169,6 @@ static int upload_tables(awp_batch *b)
         b->max_kept = std::max(b->max_kept, c->nkept);
     }
     b->total = tile0;
-    b->fs_total = fs0;
     if (b->split)
         BTRY(b, hipMemcpyAsync(b->d_sjobs, sj.data(), n * sizeof(SJob), hipMemcpyHostToDevice, b->stream));
     else
@@ -196,7 +194,7 @@ static hipError_t launch_kernels(awp_batch *b, int par)
 {
     const int n = (int)b->runs.size();
     if (b->split)
-        return launch_step_split_batch(b->mixed, b->l, b->o32, b->d_sjobs, n, b->total, b->fs_total,
+        return launch_step_split_batch(b->mixed, b->l, b->o32, b->d_sjobs, n, b->total,
                                        b->grid_v, b->grid_s, b->persist && b->claims ? b->d_claim : nullptr,
                                        b->stream);
     return launch_step_fused_batch(b->mixed, b->l, b->d_jobs, n, b->total, b->grid, par, b->d_claim, b->stream);

@@ -348,7 +348,7 @@ extern "C" int awp_create(awp_ctx **out, const awp_in3d *p, int device, int stor
     ctx->d_claim = nullptr;
     ctx->d_fjob = nullptr;
     ctx->fgrid = ctx->ftotal = 0;
-    ctx->split_total = ctx->split_fs = 0;
+    ctx->split_total = 0;
     ctx->sgrid_v = ctx->sgrid_s = 0;
     ctx->npsrc = 0;
     ctx->d_psrc = ctx->d_ptop = nullptr;
@@ -775,9 +775,8 @@ static int upload_sjob(awp_ctx *ctx)
 {
     HIPTRY(ctx, hipStreamSynchronize(ctx->stream));
     if (!ctx->d_sjob) HIPTRY(ctx, hipMalloc((void **)&ctx->d_sjob, sizeof(SJob)));
-    const SJob q = split_job(ctx->g, ctx->view(ctx->cur), ctx->c, ctx->l, 0, 0);
+    const SJob q = split_job(ctx->g, ctx->view(ctx->cur), ctx->c, ctx->l, 0);
     ctx->split_total = split_tiles(q);
-    ctx->split_fs = split_fs_blocks(q);
     awp::split_batch_grids(ctx->mixed(), ctx->l, ctx->device, &ctx->sgrid_v, &ctx->sgrid_s);
     HIPTRY(ctx, hipMemcpy(ctx->d_sjob, &q, sizeof(SJob), hipMemcpyHostToDevice));
     return AWP_OK;
@@ -815,7 +814,6 @@ static int split_launch(awp_ctx *ctx, hipStream_t st, hipEvent_t *e)
     HIPTRY(ctx, awp::launch_split_velocity(ctx->mixed(), ctx->l, ctx->l.o32, ctx->d_sjob, 1, ctx->split_total, gv,
                                            claim, st));
     if (e) HIPTRY(ctx, hipEventRecord(e[1], st));
-    HIPTRY(ctx, awp::launch_split_fs(ctx->mixed(), ctx->d_sjob, 1, ctx->split_fs, st));
     if (e) HIPTRY(ctx, hipEventRecord(e[2], st));
     HIPTRY(ctx, awp::launch_split_stress(ctx->mixed(), ctx->l, ctx->l.o32, ctx->d_sjob, 1, ctx->split_total, gs,
                                          claim, st));

@@ -37,7 +37,7 @@ struct awp_ctx {
     bool fused;              // the step in use: fused one-sweep (true) or two-stage
     bool two_bufs;           // the allocation holds wf[1] (the fused step can run)
     // the two-stage step's job table (one entry: this run), uploaded by
-    // awp_init, and its tile and free-surface block counts
+    // awp_init, and its tile count
     awp::SJob *d_sjob;
     // the claimed fused step's one-entry job table (both buffers), its
     // persistent grid and tile claim counters (CLAIM_WORDS, zero between
@@ -45,7 +45,7 @@ struct awp_ctx {
     awp::FJob *d_fjob;
     int fgrid, ftotal;
     unsigned long long *d_claim;
-    int split_total, split_fs;
+    int split_total;
     int sgrid_v, sgrid_s;    // the two-stage kernels' persistent grids (claimed launches)
     float *prof;             // fx | fy | fz
     // the per-step job-value trace (CHKJ, pmcl3d.f:1476-1479): u1 v1 w1 at

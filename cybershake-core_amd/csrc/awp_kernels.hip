@@ -186,53 +186,49 @@ __device__ __forceinline__ void velocity_tile_b(const Geo &g, const State &s0, c
 }
 
 // ---------------------------------------------------------------------------
-// free-surface velocity images: fvelxy then fvelz (operator.f:246-306).
-// u(i+1), v(j-1) at nz+1 are recomputed from the same inputs fvelxy uses,
-// so no thread reads another thread's output.
+// free-surface velocity images of column (i, j): fvelxy then fvelz
+// (operator.f:246-306) from the new velocities of level nz (and w at nz-1).
+// u(i+1), v(j-1) at nz+1 are recomputed from the same inputs fvelxy uses, so
+// no thread reads another thread's image; only the stress update of the
+// column itself reads them, so its own thread makes and stores them (a
+// kernel of their own cost 4.9 us a step, of 21 at 48x40x32).
 // ---------------------------------------------------------------------------
-template <class P>
-__device__ __forceinline__ void fs_velocity_block(const Geo &g, const State &s0, const int bx, const int by)
+// at(array, di, dj, dk): an array's value at the given offsets from (i, j, nz)
+template <class P, class AT>
+__device__ __forceinline__ void fs_images(const Geo &g, const GState &s, const int i, const int j, AT at, float &ut,
+                                          float &vt, float &wt)
 {
-    const GState s = as_global(s0);
-    const int i = bx * TX + threadIdx.x + 1;
-    const int j = by * blockDim.y + threadIdx.y + 1;
-    if (i > g.nx || j > g.ny) return;
-    const long long sy = g.sy, sz = g.sz;
-    const long long p = gidx(g, i, j, g.nz);
-    const long long q = p + sz;
     const G<float> *u1 = s.u1, *v1 = s.v1, *w1 = s.w1;
-    const float w0 = w1[p];
-    const float ut = u1[p] - (w0 - w1[p - 1]);
-    const float vt = v1[p] - (w1[p + sy] - w0);
-    const float ut_ip1 = (i < g.nx) ? (u1[p + 1] - (w1[p + 1] - w0)) : 0.0f;
-    const float vt_jm1 = (j > 1) ? (v1[p - sy] - (w0 - w1[p - sy])) : 0.0f;
+    const float u0 = at(u1, 0, 0, 0), v0 = at(v1, 0, 0, 0), w0 = at(w1, 0, 0, 0);
+    const float u_ip1 = at(u1, 1, 0, 0), v_jm1 = at(v1, 0, -1, 0);
+    ut = u0 - (w0 - at(w1, -1, 0, 0));
+    vt = v0 - (at(w1, 0, 1, 0) - w0);
+    const float ut_ip1 = (i < g.nx) ? (u_ip1 - (at(w1, 1, 0, 0) - w0)) : 0.0f;
+    const float vt_jm1 = (j > 1) ? (v_jm1 - (w0 - at(w1, 0, -1, 0))) : 0.0f;
     using M = typename P::M;
     const float mb = P::mixed ? s.mbar[mbar_idx(g, 1, g.nz)] : 0.0f;
     const float lb = P::mixed ? s.mbar[mbar_idx(g, 2, g.nz)] : 0.0f;
     float xl, xm;
     if constexpr (P::mixed) {
-        const unsigned w = ((const G<unsigned> *)s.mu)[p];   // (mu, lam) pair
+        const unsigned w = at((const G<unsigned> *)s.mu, 0, 0, 0);   // (mu, lam) pair
         xl = 1.0f / mdec(h_hi(w), lb);
         xm = 2.0f / mdec(h_lo(w), mb);
     } else {
-        xl = 1.0f / mdec(((const G<M> *)s.lam)[p], lb);
-        xm = 2.0f / mdec(((const G<M> *)s.mu)[p], mb);
+        xl = 1.0f / mdec(at((const G<M> *)s.lam, 0, 0, 0), lb);
+        xm = 2.0f / mdec(at((const G<M> *)s.mu, 0, 0, 0), mb);
     }
     const float xl2m = xm + xl;
-    const float wt = w1[p - sz] - (xl / xl2m) * (
+    wt = at(w1, 0, 0, -1) - (xl / xl2m) * (
         (ut_ip1 - ut) +
-        (u1[p + 1] - u1[p]) +
+        (u_ip1 - u0) +
         (vt - vt_jm1) +
-        (v1[p] - v1[p - sy]));
-    s.u1[q] = ut;
-    s.v1[q] = vt;
-    s.w1[q] = wt;
+        (v0 - v_jm1));
 }
 
 // ---------------------------------------------------------------------------
 // stress + memory variables: allq (viscoop.f:49-191) fused with addcrjstr
-// (cerjan.f:249-290) and, in the block that reaches k = nz, fstr
-// (operator.f:575-612).
+// (cerjan.f:249-290) and, in the block that reaches k = nz, fvelxy, fvelz and
+// fstr (operator.f:246-306, 575-612).
 // ---------------------------------------------------------------------------
 // Two forms of the same statements: stress_tile_e addresses the arrays with
 // 64-bit element indices (any size), stress_tile_b through a 32-bit byte
@@ -269,9 +265,9 @@ __device__ __forceinline__ void stress_tile_e(const Geo &g, const State &s0, con
     const long long sy = g.sy, sz = g.sz;
     long long o = g.base + (long long)kb * sz + (long long)j * sy + i;
 
-    const G<float> *__restrict__ u1 = s.u1;
-    const G<float> *__restrict__ v1 = s.v1;
-    const G<float> *__restrict__ w1 = s.w1;
+    const G<float> *u1 = s.u1;
+    const G<float> *v1 = s.v1;
+    const G<float> *w1 = s.w1;
     using M = typename P::M;
     const G<M> *__restrict__ lam = (const G<M> *)s.lam;
     const G<M> *__restrict__ mu = (const G<M> *)s.mu;
@@ -326,8 +322,8 @@ __device__ __forceinline__ void stress_tile_e(const Geo &g, const State &s0, con
 
 #pragma unroll U
     for (int k = kb; k <= ke; ++k, o += sz) {
-        const float u_p2 = u1[o + 2 * sz];
-        const float v_p2 = v1[o + 2 * sz];
+        float u_p2 = u1[o + 2 * sz];
+        float v_p2 = v1[o + 2 * sz];
         const float w_p1 = w1[o + sz];
         const float mb = P::mixed ? s.mbar[mbar_idx(g, 1, k)] : 0.0f;
         const float lb = P::mixed ? s.mbar[mbar_idx(g, 2, k)] : 0.0f;
@@ -357,6 +353,19 @@ __device__ __forceinline__ void stress_tile_e(const Geo &g, const State &s0, con
         const float w_im1 = w1[o - 1], w_ip1 = w1[o + 1], w_im2 = w1[o - 2];
         const float w_jp1 = w1[o + sy], w_jp2 = w1[o + 2 * sy], w_jm1 = w1[o - sy];
 
+        if (k == g.nz - 1) {
+            // the images at nz+1 (the top chunk spans at least three levels,
+            // so this level is met before any that reads them)
+            float ut, vt, wt;
+            fs_images<P>(g, s, i, j, [&](const auto *a, int di, int dj, int dk) { return a[o + sz + di + dj * sy + dk * sz]; }, ut, vt, wt);
+            u_p2 = ut;
+            v_p2 = vt;
+            if (act) {
+                s.u1[o + 2 * sz] = ut;
+                s.v1[o + 2 * sz] = vt;
+                s.w1[o + 2 * sz] = wt;   // read back as w_p1 at k = nz
+            }
+        }
         const bool odd = (((g.nz + 1) - k) & 1) != 0;
         const float vx1 = odd ? t1o : t1e;
         const float vx2 = odd ? t2o : t2e;
@@ -508,9 +517,9 @@ __device__ __forceinline__ void stress_tile_b(const Geo &g, const State &s0, con
     Cursor32 p(g, g.base + (long long)kb * g.sz + (long long)j * g.sy + i);
     using O = unsigned;
 
-    const G<float> *__restrict__ u1 = s.u1;
-    const G<float> *__restrict__ v1 = s.v1;
-    const G<float> *__restrict__ w1 = s.w1;
+    const G<float> *u1 = s.u1;
+    const G<float> *v1 = s.v1;
+    const G<float> *w1 = s.w1;
     using M = typename P::M;
     const G<M> *__restrict__ lam = (const G<M> *)s.lam;
     const G<M> *__restrict__ mu = (const G<M> *)s.mu;
@@ -571,8 +580,8 @@ __device__ __forceinline__ void stress_tile_b(const Geo &g, const State &s0, con
 
 #pragma unroll U
     for (int k = kb; k <= ke; ++k, p.up(), xo += xstep) {
-        const float u_p2 = p.ld(u1, 0, 0, 2);
-        const float v_p2 = p.ld(v1, 0, 0, 2);
+        float u_p2 = p.ld(u1, 0, 0, 2);
+        float v_p2 = p.ld(v1, 0, 0, 2);
         const float w_p1 = p.ld(w1, 0, 0, 1);
         const float mb = P::mixed ? s.mbar[mbar_idx(g, 1, k)] : 0.0f;
         const float lb = P::mixed ? s.mbar[mbar_idx(g, 2, k)] : 0.0f;
@@ -604,6 +613,19 @@ __device__ __forceinline__ void stress_tile_b(const Geo &g, const State &s0, con
         const float w_im1 = p.ld(w1, -1), w_ip1 = p.ld(w1, 1), w_im2 = p.ld(w1, -2);
         const float w_jp1 = p.ld(w1, 0, 1), w_jp2 = p.ld(w1, 0, 2), w_jm1 = p.ld(w1, 0, -1);
 
+        if (k == g.nz - 1) {
+            // the images at nz+1 (the top chunk spans at least three levels,
+            // so this level is met before any that reads them)
+            float ut, vt, wt;
+            fs_images<P>(g, s, i, j, [&](const auto *a, int di, int dj, int dk) { return p.ld(a, di, dj, dk + 1); }, ut, vt, wt);
+            u_p2 = ut;
+            v_p2 = vt;
+            if (act) {
+                p.st(s.u1, ut, 0, 0, 2);
+                p.st(s.v1, vt, 0, 0, 2);
+                p.st(s.w1, wt, 0, 0, 2);   // read back as w_p1 at k = nz
+            }
+        }
         const bool odd = (((g.nz + 1) - k) & 1) != 0;
         const float vx1 = odd ? t1o : t1e;
         const float vx2 = odd ? t2o : t2e;
@@ -819,21 +841,6 @@ k_stress_batch(const SJob *__restrict__ jobs, const int njobs, const int total, 
         stress_tile<P, U, O32>(J.g, J.s, J.c, J.kc, bx, by, bz);
     }
     if (claim && threadIdx.x == 0 && threadIdx.y == 0 && threadIdx.z == 0) claim_done(claim, (int)gridDim.x);
-}
-
-// free-surface images of every run: block b of the launch is block
-// b - fs0 of its run's (nx/64) x (ny/4) surface grid
-template <class P>
-__global__ void __launch_bounds__(256)
-k_fs_velocity_batch(const SJob *__restrict__ jobs, const int njobs)
-{
-    const int b = blockIdx.x;
-    int jb = 0;
-    while (jb + 1 < njobs && jobs[jb + 1].fs0 <= b) ++jb;
-    const SJob &J = jobs[jb];
-    const int lb = b - J.fs0;
-    const int fnx = (J.g.nx + TX - 1) / TX;
-    fs_velocity_block<P>(J.g, J.s, lb % fnx, lb / fnx);
 }
 
 // ---------------------------------------------------------------------------
@@ -1504,16 +1511,6 @@ hipError_t launch_split_velocity(bool mixed, const Launch &l, bool o32, const SJ
     return hipGetLastError();
 }
 
-hipError_t launch_split_fs(bool mixed, const SJob *d_jobs, int njobs, int fs_total, hipStream_t st)
-{
-    if (njobs <= 0 || fs_total <= 0) return hipSuccess;
-    if (mixed)
-        hipLaunchKernelGGL(k_fs_velocity_batch<StoreMixed>, dim3(fs_total), dim3(TX, 4), 0, st, d_jobs, njobs);
-    else
-        hipLaunchKernelGGL(k_fs_velocity_batch<StoreF32>, dim3(fs_total), dim3(TX, 4), 0, st, d_jobs, njobs);
-    return hipGetLastError();
-}
-
 hipError_t launch_split_stress(bool mixed, const Launch &l, bool o32, const SJob *d_jobs, int njobs, int total,
                                int grid_s, unsigned long long *claim, hipStream_t st)
 {
@@ -1527,11 +1524,10 @@ hipError_t launch_split_stress(bool mixed, const Launch &l, bool o32, const SJob
 }
 
 hipError_t launch_step_split_batch(bool mixed, const Launch &l, bool o32, const SJob *d_jobs, int njobs,
-                                   int total, int fs_total, int grid_v, int grid_s, unsigned long long *claim,
+                                   int total, int grid_v, int grid_s, unsigned long long *claim,
                                    hipStream_t st)
 {
     hipError_t e = launch_split_velocity(mixed, l, o32, d_jobs, njobs, total, grid_v, claim, st);
-    if (e == hipSuccess) e = launch_split_fs(mixed, d_jobs, njobs, fs_total, st);
     if (e == hipSuccess) e = launch_split_stress(mixed, l, o32, d_jobs, njobs, total, grid_s, claim, st);
     return e;
 }

@@ -636,12 +636,10 @@ struct SJob {
     int kc;
     int nbx, nby, nbz;
     int tile0;   // first global tile of the run (velocity and stress stages)
-    int fs0;     // first block of the run in the free-surface launch
     int pw, ph;  // tile patches (patch_tile); pw = nbx, ph = 1 is row order
 };
-// The job of one run, its tiles numbered from tile0 and its free-surface
-// blocks from fs0.
-static inline SJob split_job(const Geo &g, const State &s, const Coef &c, const Launch &l, int tile0, int fs0)
+// The job of one run, its tiles numbered from tile0.
+static inline SJob split_job(const Geo &g, const State &s, const Coef &c, const Launch &l, int tile0)
 {
     SJob q;
     q.g = g;
@@ -652,27 +650,23 @@ static inline SJob split_job(const Geo &g, const State &s, const Coef &c, const 
     q.nby = (g.ny + l.tile_y - 1) / l.tile_y;
     q.nbz = l.nchunk;
     q.tile0 = tile0;
-    q.fs0 = fs0;
     q.pw = l.spw > 0 ? (l.spw < q.nbx ? l.spw : q.nbx) : q.nbx;
     q.ph = l.sph > 0 ? l.sph : 1;
     return q;
 }
 static inline int split_tiles(const SJob &q) { return q.nbx * q.nby * q.nbz; }
-static inline int split_fs_blocks(const SJob &q) { return ((q.g.nx + TX - 1) / TX) * ((q.g.ny + 3) / 4); }
 
-// velocity, free-surface and stress stages of every run: three launches,
-// the first and last over the tile list (grid_v / grid_s blocks, from
-// split_batch_grids, or one block per tile when larger); fs_total = sum of
-// the runs' free-surface blocks; o32 = offsets32() holds for every run.
+// velocity and stress stages of every run: two launches over the tile list
+// (grid_v / grid_s blocks, from split_batch_grids, or one block per tile when
+// larger); o32 = offsets32() holds for every run.
 // With `claim` (CLAIM_WORDS words, zero before the first launch, left zero
 // by each; launches sharing it must not overlap) the blocks claim tiles per
 // XCD (claim_tile, ranges rotated by l.xrot); without, the static walk.
 hipError_t launch_step_split_batch(bool mixed, const Launch &l, bool o32, const SJob *d_jobs, int njobs,
-                                   int total, int fs_total, int grid_v, int grid_s, unsigned long long *claim,
+                                   int total, int grid_v, int grid_s, unsigned long long *claim,
                                    hipStream_t st);
 hipError_t launch_split_velocity(bool mixed, const Launch &l, bool o32, const SJob *d_jobs, int njobs, int total,
                                  int grid_v, unsigned long long *claim, hipStream_t st);
-hipError_t launch_split_fs(bool mixed, const SJob *d_jobs, int njobs, int fs_total, hipStream_t st);
 hipError_t launch_split_stress(bool mixed, const Launch &l, bool o32, const SJob *d_jobs, int njobs, int total,
                                int grid_s, unsigned long long *claim, hipStream_t st);
 void split_batch_grids(bool mixed, const Launch &l, int device, int *grid_v, int *grid_s);
