@@ -704,6 +704,9 @@ extern "C" int awp_set_source(awp_ctx *ctx, int nsrc, const int *xyz, const floa
     HIPTRY(ctx, hipMemcpy(ctx->d_ptop, top.data(), nsrc * sizeof(long long), hipMemcpyHostToDevice));
     HIPTRY(ctx, hipMemcpy(ctx->d_stf, stf, ns * sizeof(float), hipMemcpyHostToDevice));
     ctx->npsrc = nsrc;
+    ctx->src_ijk[0] = xyz[0];
+    ctx->src_ijk[1] = xyz[1];
+    ctx->src_ijk[2] = p.nz + 1 - xyz[2];
     ctx->source_set = true;
     ctx->initialised = false;
     return AWP_OK;
@@ -804,19 +807,20 @@ static int upload_fjob(awp_ctx *ctx)
 }
 
 // the two-stage step's kernels in buffer 0: claimed (persistent blocks) or
-// one block per tile; e: the timing events of the step, or null
-static int split_launch(awp_ctx *ctx, hipStream_t st, hipEvent_t *e)
+// one block per tile; e: the timing events of the step, or null; hv, hs: the
+// source and trace work the velocity and the stress kernel do on the way
+static int split_launch(awp_ctx *ctx, hipStream_t st, hipEvent_t *e, const awp::Hook &hv, const awp::Hook &hs)
 {
     const bool cl = ctx->l.claim == 2 ||
                     (ctx->l.claim == 1 && ctx->split_total >= 4 * std::max(ctx->sgrid_v, ctx->sgrid_s));
     const int gv = cl ? ctx->sgrid_v : 1 << 30, gs = cl ? ctx->sgrid_s : 1 << 30;
     unsigned long long *claim = cl ? ctx->d_claim : nullptr;
     HIPTRY(ctx, awp::launch_split_velocity(ctx->mixed(), ctx->l, ctx->l.o32, ctx->d_sjob, 1, ctx->split_total, gv,
-                                           claim, st));
+                                           claim, hv, st));
     if (e) HIPTRY(ctx, hipEventRecord(e[1], st));
     if (e) HIPTRY(ctx, hipEventRecord(e[2], st));
     HIPTRY(ctx, awp::launch_split_stress(ctx->mixed(), ctx->l, ctx->l.o32, ctx->d_sjob, 1, ctx->split_total, gs,
-                                         claim, st));
+                                         claim, hs, st));
     return AWP_OK;
 }
 
@@ -908,6 +912,29 @@ extern "C" int awp_step(awp_ctx *ctx, int nsteps)
         int rc = scheme_changed(ctx);
         if (rc) return rc;
     }
+    // One source, two-stage: the step kernels themselves apply its samples
+    // and take the trace rows between the steps of this call (Hook); only the
+    // last step's are left to k_source.
+    const bool hooked = !ctx->fused && ctx->npsrc == 1;
+    auto hook_of = [ctx, &p](int sample, int row) {
+        awp::Hook h = {};
+        h.vtst = ctx->vtst;
+        h.vtst1 = ctx->vtst1;
+        if (sample >= 1 && sample <= p.nst) {
+            h.kind = p.igreen;
+            h.i = ctx->src_ijk[0];
+            h.j = ctx->src_ijk[1];
+            h.k = ctx->src_ijk[2];
+            h.amp = ctx->d_stf + (size_t)(sample - 1) * 6;
+        }
+        if (row >= 0) {
+            h.trace = ctx->d_trace + 3 * (size_t)row;
+            h.ti = ctx->trace_ijk[0];
+            h.tj = ctx->trace_ijk[1];
+            h.tk = ctx->trace_ijk[2];
+        }
+        return h;
+    };
     for (int n = 0; n < todo; ++n) {
         const int i = ++ctx->step;
         hipEvent_t *e = ctx->timing ? &ctx->ev[(size_t)6 * n] : nullptr;
@@ -925,13 +952,20 @@ extern "C" int awp_step(awp_ctx *ctx, int nsteps)
             // the stage kernels over this run's one-entry job table (in
             // buffer 0)
             sn = ctx->view(ctx->cur);
-            int rc = split_launch(ctx, st, e);
+            // before step i of this call: sample i of a body force and the
+            // trace row of step i - 1; after it: sample i + 1 of a surface source
+            const bool body = p.igreen <= 3;
+            const awp::Hook hv = hooked && n > 0 ? hook_of(body ? i : 0, i - 2) : awp::Hook{};
+            const awp::Hook hs = hooked && !body ? hook_of(i + 1, -1) : awp::Hook{};
+            int rc = split_launch(ctx, st, e, hv, hs);
             if (rc) return rc;
         }
         if (e) HIPTRY(ctx, hipEventRecord(e[3], st));
         // source sample i + 1 (while the source lasts), then the trace row
-        HIPTRY(ctx, launch_source(ctx->g, sn, p.igreen, ctx->npsrc, ctx->d_psrc, ctx->d_ptop, ctx->d_stf, p.nst,
-                                  i + 1, ctx->vtst, ctx->vtst1, i + 1 <= p.nst, ctx->d_trace, ctx->trace_pos, st));
+        if (!hooked || n == todo - 1)
+            HIPTRY(ctx, launch_source(ctx->g, sn, p.igreen, ctx->npsrc, ctx->d_psrc, ctx->d_ptop, ctx->d_stf, p.nst,
+                                      i + 1, ctx->vtst, ctx->vtst1, i + 1 <= p.nst && (!hooked || p.igreen <= 3),
+                                      ctx->d_trace, ctx->trace_pos, st));
         if (i % p.ntiskp_sgt == 0 && ctx->nsamp < ctx->nsamp_max) {
             HIPTRY(ctx, launch_sgt_gather(sn, ctx->nkept, ctx->d_kpos, ctx->d_kidx, ctx->d_sg, ctx->d_sgt,
                                           ctx->nsamp_max, ctx->nsamp, st));
@@ -989,7 +1023,7 @@ int trial_steps(awp_ctx *ctx, int n)
             HIPTRY(ctx, fused_launch(ctx, ctx->stream));
             ctx->cur ^= 1;
         } else {
-            int rc = split_launch(ctx, ctx->stream, nullptr);
+            int rc = split_launch(ctx, ctx->stream, nullptr, awp::Hook{}, awp::Hook{});
             if (rc) return rc;
         }
     }

@@ -55,6 +55,7 @@ struct awp_ctx {
     int trace_ijk[3];
     // sources
     int npsrc;
+    int src_ijk[3];          // the first source's node
     long long *d_psrc;       // [npsrc] node index
     long long *d_ptop;       // [npsrc] index of (x, y, nz)
     float *d_stf;            // [npsrc][nst][6]

@@ -22,13 +22,33 @@
 
 namespace awp {
 
+// The pending body-force sample and trace row (Hook) at node (i, j, k), whose
+// density is d, before the node's velocity update: addsrc (source.f:812-913)
+// and the trace of pmcl3d.f:1476-1479, as k_source does them.
+__device__ __forceinline__ void hook_velocity(const Hook &h, const int i, const int j, const int k, const float d,
+                                              float &u, float &v, float &w)
+{
+    if (k == h.k && i == h.i && j == h.j && h.kind >= 1 && h.kind <= 3) {
+        const float amp = h.amp[h.kind - 1];
+        const float add = amp * h.vtst / d;
+        u = h.kind == 1 ? u + add : u;
+        v = h.kind == 2 ? v + add : v;
+        w = h.kind == 3 ? w + add : w;
+    }
+    if (h.trace && k == h.tk && i == h.ti && j == h.tj) {
+        h.trace[0] = u;
+        h.trace[1] = v;
+        h.trace[2] = w;
+    }
+}
+
 // ---------------------------------------------------------------------------
 // velocity: uxx1/vyy1/wzz1 (operator.f:92-244) fused with addcrjvel
 // (cerjan.f:292-328)
 // ---------------------------------------------------------------------------
 template <class P, int U>
 __device__ __forceinline__ void velocity_tile(const Geo &g, const State &s0, const Coef &c, const int kc, const int bx,
-                                     const int by, const int bz)
+                                     const int by, const int bz, const Hook &hook)
 {
     const GState s = as_global(s0);
     using M = typename P::M;
@@ -73,23 +93,25 @@ __device__ __forceinline__ void velocity_tile(const Geo &g, const State &s0, con
         const float yy_0 = yy[o], yy_jp1 = yy[o + sy], yy_jp2 = yy[o + 2 * sy], yy_jm1 = yy[o - sy];
         const float xz_ip1 = xz[o + 1], xz_ip2 = xz[o + 2], xz_im1 = xz[o - 1];
         const float yz_jm1 = yz[o - sy], yz_jp1 = yz[o + sy], yz_jm2 = yz[o - 2 * sy];
+        float u0 = nt_ld(&s.u1[o]), v0 = nt_ld(&s.v1[o]), w0 = nt_ld(&s.w1[o]);
+        if (k == hook.k || k == hook.tk) hook_velocity(hook, i, j, k, dA, u0, v0, w0);
 
         float d, q, u, v, w;
         d = 0.25f * ((dA + dB) + (dA_m + dB_m));
         q = dth / d;
-        u = nt_ld(&s.u1[o]) + q * (
+        u = u0 + q * (
             c1 * (xx_0 - xx_m1) + c2 * (xx_p1 - xx_m2) +
             c1 * (xy_0 - xy_jm1) + c2 * (xy_jp1 - xy_jm2) +
             c1 * (xz_0 - xz_m1) + c2 * (xz_p1 - xz_m2));
         d = 0.25f * ((dA + dC) + (dA_m + dC_m));
         q = dth / d;
-        v = nt_ld(&s.v1[o]) + q * (
+        v = v0 + q * (
             c1 * (xy_ip1 - xy_0) + c2 * (xy_ip2 - xy_im1) +
             c1 * (yy_jp1 - yy_0) + c2 * (yy_jp2 - yy_jm1) +
             c1 * (yz_0 - yz_m1) + c2 * (yz_p1 - yz_m2));
         d = 0.25f * ((dA + dC) + (dB + dD));
         q = dth / d;
-        w = nt_ld(&s.w1[o]) + q * (
+        w = w0 + q * (
             c1 * (xz_ip1 - xz_0) + c2 * (xz_ip2 - xz_im1) +
             c1 * (yz_0 - yz_jm1) + c2 * (yz_jp1 - yz_jm2) +
             c1 * (zz_p1 - zz_0) + c2 * (zz_p2 - zz_m1));
@@ -110,7 +132,7 @@ __device__ __forceinline__ void velocity_tile(const Geo &g, const State &s0, con
 // below 4 GiB.
 template <class P, int U>
 __device__ __forceinline__ void velocity_tile_b(const Geo &g, const State &s0, const Coef &c, const int kc, const int bx,
-                                       const int by, const int bz)
+                                       const int by, const int bz, const Hook &hook)
 {
     const GState s = as_global(s0);
     const int i = (bx * blockDim.z + threadIdx.z) * TX + threadIdx.x + 1;
@@ -153,23 +175,25 @@ __device__ __forceinline__ void velocity_tile_b(const Geo &g, const State &s0, c
         const float yy_0 = p.ld(yy), yy_jp1 = p.ld(yy, 0, 1), yy_jp2 = p.ld(yy, 0, 2), yy_jm1 = p.ld(yy, 0, -1);
         const float xz_ip1 = p.ld(xz, 1), xz_ip2 = p.ld(xz, 2), xz_im1 = p.ld(xz, -1);
         const float yz_jm1 = p.ld(yz, 0, -1), yz_jp1 = p.ld(yz, 0, 1), yz_jm2 = p.ld(yz, 0, -2);
+        float u0 = p.ldn(s.u1), v0 = p.ldn(s.v1), w0 = p.ldn(s.w1);
+        if (k == hook.k || k == hook.tk) hook_velocity(hook, i, j, k, dA, u0, v0, w0);
 
         float d, q, u, v, w;
         d = 0.25f * ((dA + dB) + (dA_m + dB_m));
         q = dth / d;
-        u = p.ldn(s.u1) + q * (
+        u = u0 + q * (
             c1 * (xx_0 - xx_m1) + c2 * (xx_p1 - xx_m2) +
             c1 * (xy_0 - xy_jm1) + c2 * (xy_jp1 - xy_jm2) +
             c1 * (xz_0 - xz_m1) + c2 * (xz_p1 - xz_m2));
         d = 0.25f * ((dA + dC) + (dA_m + dC_m));
         q = dth / d;
-        v = p.ldn(s.v1) + q * (
+        v = v0 + q * (
             c1 * (xy_ip1 - xy_0) + c2 * (xy_ip2 - xy_im1) +
             c1 * (yy_jp1 - yy_0) + c2 * (yy_jp2 - yy_jm1) +
             c1 * (yz_0 - yz_m1) + c2 * (yz_p1 - yz_m2));
         d = 0.25f * ((dA + dC) + (dB + dD));
         q = dth / d;
-        w = p.ldn(s.w1) + q * (
+        w = w0 + q * (
             c1 * (xz_ip1 - xz_0) + c2 * (xz_ip2 - xz_im1) +
             c1 * (yz_0 - yz_jm1) + c2 * (yz_jp1 - yz_jm2) +
             c1 * (zz_p1 - zz_0) + c2 * (zz_p2 - zz_m1));
@@ -226,6 +250,28 @@ __device__ __forceinline__ void fs_images(const Geo &g, const GState &s, const i
 }
 
 // ---------------------------------------------------------------------------
+// A surface source's sample (Hook, igreen 4..6; source.f:870-902) at column
+// (i, j), after its thread wrote level nz and the images above: at(a, dk) and
+// put(a, v, dk) access an array at nz + dk.
+// ---------------------------------------------------------------------------
+template <class AT, class PUT>
+__device__ __forceinline__ void hook_stress(const Hook &h, const GState &s, const int i, const int j, AT at, PUT put)
+{
+    if (h.kind < 4 || i != h.i || j != h.j) return;
+    if (h.kind == 6) {
+        const float a = h.amp[2];
+        put(s.zz, 2.0f * a * h.vtst1 - at(s.zz, 0), 1);
+        put(s.zz, 2.0f * a * h.vtst1 - at(s.zz, -1), 2);
+    } else {
+        G<float> *f = h.kind == 4 ? s.xz : s.yz;
+        const float a = h.amp[h.kind - 4];
+        put(f, a * h.vtst1, 0);
+        put(f, 2.0f * a * h.vtst1 - at(f, -1), 1);
+        put(f, 2.0f * a * h.vtst1 - at(f, -2), 2);
+    }
+}
+
+// ---------------------------------------------------------------------------
 // stress + memory variables: allq (viscoop.f:49-191) fused with addcrjstr
 // (cerjan.f:249-290) and, in the block that reaches k = nz, fvelxy, fvelz and
 // fstr (operator.f:246-306, 575-612).
@@ -240,7 +286,7 @@ __device__ __forceinline__ void fs_images(const Geo &g, const GState &s, const i
 // kernel.
 template <class P, int U>
 __device__ __forceinline__ void stress_tile_e(const Geo &g, const State &s0, const Coef &c, const int kc, const int bx,
-                                   const int by, const int bz)
+                                   const int by, const int bz, const Hook &hook)
 {
     const GState s = as_global(s0);
     using Q = typename P::Q;
@@ -472,6 +518,8 @@ __device__ __forceinline__ void stress_tile_e(const Geo &g, const State &s0, con
             s.xz[o + 2 * sz] = -xz_f2;
             s.yz[o + sz] = -yz_f1;
             s.yz[o + 2 * sz] = -yz_f2;
+            hook_stress(hook, s, i, j, [&](const auto *a, int dk) { return a[o + dk * sz]; },
+                        [&](auto *a, float v, int dk) { a[o + dk * sz] = v; });
         } else {
             s.zz[o] = zz; s.xz[o] = xz; s.yz[o] = yz;
         }
@@ -492,7 +540,7 @@ __device__ __forceinline__ void stress_tile_e(const Geo &g, const State &s0, con
 
 template <class P, int U>
 __device__ __forceinline__ void stress_tile_b(const Geo &g, const State &s0, const Coef &c, const int kc, const int bx,
-                                   const int by, const int bz)
+                                   const int by, const int bz, const Hook &hook)
 {
     const GState s = as_global(s0);
     using Q = typename P::Q;
@@ -734,6 +782,8 @@ __device__ __forceinline__ void stress_tile_b(const Geo &g, const State &s0, con
                 p.st(s.xz, -xz_f2, 0, 0, 2);
                 p.st(s.yz, -yz_f1, 0, 0, 1);
                 p.st(s.yz, -yz_f2, 0, 0, 2);
+                hook_stress(hook, s, i, j, [&](const auto *a, int dk) { return p.ld(a, 0, 0, dk); },
+                            [&](auto *a, float v, int dk) { p.st(a, v, 0, 0, dk); });
             } else {
                 p.stn(s.zz, zz); p.stn(s.xz, xz); p.stn(s.yz, yz);
             }
@@ -754,12 +804,12 @@ __device__ __forceinline__ void stress_tile_b(const Geo &g, const State &s0, con
 
 template <class P, int U, bool O32>
 __device__ __forceinline__ void stress_tile(const Geo &g, const State &s0, const Coef &c, const int kc, const int bx,
-                                   const int by, const int bz)
+                                   const int by, const int bz, const Hook &hook)
 {
     if constexpr (O32)
-        stress_tile_b<P, U>(g, s0, c, kc, bx, by, bz);
+        stress_tile_b<P, U>(g, s0, c, kc, bx, by, bz, hook);
     else
-        stress_tile_e<P, U>(g, s0, c, kc, bx, by, bz);
+        stress_tile_e<P, U>(g, s0, c, kc, bx, by, bz, hook);
 }
 
 // ---------------------------------------------------------------------------
@@ -811,7 +861,7 @@ __device__ inline int stage_tile(unsigned long long *claim, int per, int total, 
 template <class P, int U, int MAXT, bool O32>
 __global__ void __launch_bounds__(MAXT)
 k_velocity_batch(const SJob *__restrict__ jobs, const int njobs, const int total, const int per,
-                 unsigned long long *claim, const int rot)
+                 unsigned long long *claim, const int rot, const Hook hook)
 {
     __shared__ int next;
     for (int k = 0;; ++k) {
@@ -820,9 +870,9 @@ k_velocity_batch(const SJob *__restrict__ jobs, const int njobs, const int total
         int bx, by, bz;
         const SJob &J = split_tile(jobs, njobs, tile, bx, by, bz);
         if constexpr (O32)
-            velocity_tile_b<P, U>(J.g, J.s, J.c, J.kc, bx, by, bz);
+            velocity_tile_b<P, U>(J.g, J.s, J.c, J.kc, bx, by, bz, hook);
         else
-            velocity_tile<P, U>(J.g, J.s, J.c, J.kc, bx, by, bz);
+            velocity_tile<P, U>(J.g, J.s, J.c, J.kc, bx, by, bz, hook);
     }
     if (claim && threadIdx.x == 0 && threadIdx.y == 0 && threadIdx.z == 0) claim_done(claim, (int)gridDim.x);
 }
@@ -830,7 +880,7 @@ k_velocity_batch(const SJob *__restrict__ jobs, const int njobs, const int total
 template <class P, int U, bool O32, int MAXT>
 __global__ void __launch_bounds__(MAXT)
 k_stress_batch(const SJob *__restrict__ jobs, const int njobs, const int total, const int per,
-               unsigned long long *claim, const int rot)
+               unsigned long long *claim, const int rot, const Hook hook)
 {
     __shared__ int next;
     for (int k = 0;; ++k) {
@@ -838,7 +888,7 @@ k_stress_batch(const SJob *__restrict__ jobs, const int njobs, const int total, 
         if (tile < 0) break;
         int bx, by, bz;
         const SJob &J = split_tile(jobs, njobs, tile, bx, by, bz);
-        stress_tile<P, U, O32>(J.g, J.s, J.c, J.kc, bx, by, bz);
+        stress_tile<P, U, O32>(J.g, J.s, J.c, J.kc, bx, by, bz, hook);
     }
     if (claim && threadIdx.x == 0 && threadIdx.y == 0 && threadIdx.z == 0) claim_done(claim, (int)gridDim.x);
 }
@@ -1446,79 +1496,79 @@ static int persistent_grid(int grid, int per, int total, bool claimed)
 
 template <class P, int U, int MAXT>
 static void vel_batch_t(const Launch &l, bool ov, const SJob *d_jobs, int njobs, int total, int per, int grid_v,
-                        unsigned long long *claim, hipStream_t st)
+                        unsigned long long *claim, const Hook &hook, hipStream_t st)
 {
     const dim3 grid(persistent_grid(grid_v, per, total, claim)), block(TX, l.tile_y, l.tile_xw);
     if (ov)
         hipLaunchKernelGGL((k_velocity_batch<P, U, MAXT, true>), grid, block, l.lds_v, st, d_jobs, njobs, total,
-                           per, claim, l.xrot & 7);
+                           per, claim, l.xrot & 7, hook);
     else
         hipLaunchKernelGGL((k_velocity_batch<P, U, MAXT, false>), grid, block, l.lds_v, st, d_jobs, njobs, total,
-                           per, claim, l.xrot & 7);
+                           per, claim, l.xrot & 7, hook);
 }
 
 template <class P>
 static hipError_t velocity_stage(const Launch &l, bool ov, const SJob *d_jobs, int njobs, int total, int per,
-                                 int grid_v, unsigned long long *claim, hipStream_t st)
+                                 int grid_v, unsigned long long *claim, const Hook &hook, hipStream_t st)
 {
     if (tall(l)) {
         if (l.unroll == 2) return hipErrorInvalidValue;   // no such variant
-        vel_batch_t<P, 1, 1024>(l, ov, d_jobs, njobs, total, per, grid_v, claim, st);
+        vel_batch_t<P, 1, 1024>(l, ov, d_jobs, njobs, total, per, grid_v, claim, hook, st);
     } else if (l.unroll == 2) {
-        vel_batch_t<P, 2, 512>(l, ov, d_jobs, njobs, total, per, grid_v, claim, st);
+        vel_batch_t<P, 2, 512>(l, ov, d_jobs, njobs, total, per, grid_v, claim, hook, st);
     } else {
-        vel_batch_t<P, 1, 512>(l, ov, d_jobs, njobs, total, per, grid_v, claim, st);
+        vel_batch_t<P, 1, 512>(l, ov, d_jobs, njobs, total, per, grid_v, claim, hook, st);
     }
     return hipSuccess;
 }
 
 template <class P, int U, bool O32, int MAXT>
 static void str_batch_t(const Launch &l, const SJob *d_jobs, int njobs, int total, int per, int grid_s,
-                        unsigned long long *claim, hipStream_t st)
+                        unsigned long long *claim, const Hook &hook, hipStream_t st)
 {
     hipLaunchKernelGGL((k_stress_batch<P, U, O32, MAXT>), dim3(persistent_grid(grid_s, per, total, claim)),
-                       dim3(TX, l.tile_y, l.tile_xw), l.lds_s, st, d_jobs, njobs, total, per, claim, l.xrot & 7);
+                       dim3(TX, l.tile_y, l.tile_xw), l.lds_s, st, d_jobs, njobs, total, per, claim, l.xrot & 7, hook);
 }
 
 template <class P>
 static hipError_t stress_stage(const Launch &l, bool os, const SJob *d_jobs, int njobs, int total, int per,
-                               int grid_s, unsigned long long *claim, hipStream_t st)
+                               int grid_s, unsigned long long *claim, const Hook &hook, hipStream_t st)
 {
     if (tall(l)) {
         if (!os || l.unroll == 2) return hipErrorInvalidValue;   // no such variant
-        str_batch_t<P, 1, true, 1024>(l, d_jobs, njobs, total, per, grid_s, claim, st);
+        str_batch_t<P, 1, true, 1024>(l, d_jobs, njobs, total, per, grid_s, claim, hook, st);
         return hipSuccess;
     }
     if (l.unroll == 2) {
-        if (os) str_batch_t<P, 2, true, 512>(l, d_jobs, njobs, total, per, grid_s, claim, st);
-        else str_batch_t<P, 2, false, 512>(l, d_jobs, njobs, total, per, grid_s, claim, st);
+        if (os) str_batch_t<P, 2, true, 512>(l, d_jobs, njobs, total, per, grid_s, claim, hook, st);
+        else str_batch_t<P, 2, false, 512>(l, d_jobs, njobs, total, per, grid_s, claim, hook, st);
     } else {
-        if (os) str_batch_t<P, 1, true, 512>(l, d_jobs, njobs, total, per, grid_s, claim, st);
-        else str_batch_t<P, 1, false, 512>(l, d_jobs, njobs, total, per, grid_s, claim, st);
+        if (os) str_batch_t<P, 1, true, 512>(l, d_jobs, njobs, total, per, grid_s, claim, hook, st);
+        else str_batch_t<P, 1, false, 512>(l, d_jobs, njobs, total, per, grid_s, claim, hook, st);
     }
     return hipSuccess;
 }
 
 hipError_t launch_split_velocity(bool mixed, const Launch &l, bool o32, const SJob *d_jobs, int njobs, int total,
-                                 int grid_v, unsigned long long *claim, hipStream_t st)
+                                 int grid_v, unsigned long long *claim, const Hook &hook, hipStream_t st)
 {
     if (njobs <= 0 || total <= 0) return hipSuccess;
     const int per = (total + 7) / 8;
     const bool ov = o32 && l.o32_v;
-    const hipError_t e = mixed ? velocity_stage<StoreMixed>(l, ov, d_jobs, njobs, total, per, grid_v, claim, st)
-                               : velocity_stage<StoreF32>(l, ov, d_jobs, njobs, total, per, grid_v, claim, st);
+    const hipError_t e = mixed ? velocity_stage<StoreMixed>(l, ov, d_jobs, njobs, total, per, grid_v, claim, hook, st)
+                               : velocity_stage<StoreF32>(l, ov, d_jobs, njobs, total, per, grid_v, claim, hook, st);
     if (e != hipSuccess) return e;
     return hipGetLastError();
 }
 
 hipError_t launch_split_stress(bool mixed, const Launch &l, bool o32, const SJob *d_jobs, int njobs, int total,
-                               int grid_s, unsigned long long *claim, hipStream_t st)
+                               int grid_s, unsigned long long *claim, const Hook &hook, hipStream_t st)
 {
     if (njobs <= 0 || total <= 0) return hipSuccess;
     const int per = (total + 7) / 8;
     const bool os = o32 && l.o32_s;
-    const hipError_t e = mixed ? stress_stage<StoreMixed>(l, os, d_jobs, njobs, total, per, grid_s, claim, st)
-                               : stress_stage<StoreF32>(l, os, d_jobs, njobs, total, per, grid_s, claim, st);
+    const hipError_t e = mixed ? stress_stage<StoreMixed>(l, os, d_jobs, njobs, total, per, grid_s, claim, hook, st)
+                               : stress_stage<StoreF32>(l, os, d_jobs, njobs, total, per, grid_s, claim, hook, st);
     if (e != hipSuccess) return e;
     return hipGetLastError();
 }
@@ -1527,8 +1577,9 @@ hipError_t launch_step_split_batch(bool mixed, const Launch &l, bool o32, const 
                                    int total, int grid_v, int grid_s, unsigned long long *claim,
                                    hipStream_t st)
 {
-    hipError_t e = launch_split_velocity(mixed, l, o32, d_jobs, njobs, total, grid_v, claim, st);
-    if (e == hipSuccess) e = launch_split_stress(mixed, l, o32, d_jobs, njobs, total, grid_s, claim, st);
+    const Hook none = {};
+    hipError_t e = launch_split_velocity(mixed, l, o32, d_jobs, njobs, total, grid_v, claim, none, st);
+    if (e == hipSuccess) e = launch_split_stress(mixed, l, o32, d_jobs, njobs, total, grid_s, claim, none, st);
     return e;
 }
 

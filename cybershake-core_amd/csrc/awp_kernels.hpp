@@ -656,6 +656,23 @@ static inline SJob split_job(const Geo &g, const State &s, const Coef &c, const 
 }
 static inline int split_tiles(const SJob &q) { return q.nbx * q.nby * q.nbz; }
 
+// The point source and trace work between two two-stage steps of one run with
+// one source, done by the threads that own the nodes instead of a kernel of
+// its own (4.6 us of the 17 us of a 48x40x32 step).  A body force (igreen
+// 1..3) changes one velocity, which until the next velocity update only that
+// update of the node itself reads: it is added there, and the trace row of
+// the step before is taken there too.  A surface source (igreen 4..6) sets
+// stresses of its column at the surface and above, which the column's thread
+// has just written.  Node indices 0: nothing to do.
+struct Hook {
+    int kind;              // igreen of the pending sample, 0: none
+    int i, j, k;           // the source node (k: a body force's level)
+    const float *amp;      // the sample's six values
+    float vtst, vtst1;
+    float *trace;          // row of the trace to fill, or null
+    int ti, tj, tk;        // the traced node
+};
+
 // velocity and stress stages of every run: two launches over the tile list
 // (grid_v / grid_s blocks, from split_batch_grids, or one block per tile when
 // larger); o32 = offsets32() holds for every run.
@@ -666,9 +683,9 @@ hipError_t launch_step_split_batch(bool mixed, const Launch &l, bool o32, const 
                                    int total, int grid_v, int grid_s, unsigned long long *claim,
                                    hipStream_t st);
 hipError_t launch_split_velocity(bool mixed, const Launch &l, bool o32, const SJob *d_jobs, int njobs, int total,
-                                 int grid_v, unsigned long long *claim, hipStream_t st);
+                                 int grid_v, unsigned long long *claim, const Hook &hook, hipStream_t st);
 hipError_t launch_split_stress(bool mixed, const Launch &l, bool o32, const SJob *d_jobs, int njobs, int total,
-                               int grid_s, unsigned long long *claim, hipStream_t st);
+                               int grid_s, unsigned long long *claim, const Hook &hook, hipStream_t st);
 void split_batch_grids(bool mixed, const Launch &l, int device, int *grid_v, int *grid_s);
 
 // per-run data of the batched source / SGT stage
