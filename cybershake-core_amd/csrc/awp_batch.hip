@@ -318,6 +318,12 @@ extern "C" int awp_batch_create(awp_batch **out, awp_ctx *const *runs, int nruns
         if (b->l.tile_y == 8 || (b->l.tile_y == 11 && b->l.unroll != 3)) b->l.unroll = 0;
         b->l.tile_xw = 1;
     }
+    {
+        // the cache is shared by every run of a step
+        long long nvol = 0;
+        for (int r = 0; r < nruns; ++r) nvol += runs[r]->g.nvol;
+        if (b->split && nruns > 1) b->l.cached = cache_mode(nvol, b->mixed);
+    }
     b->nchunk.assign(nruns, 1);
     // the chain of a wave's levels is hidden by every run's waves together
     {

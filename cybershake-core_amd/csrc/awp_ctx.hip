@@ -222,6 +222,10 @@ static Launch choose_launch(const Geo &g, bool fused, bool mixed, int device)
         }
     }
     l.o32 = use_o32(g);
+    // AWP_CACHED=0..3 overrides the two-stage kernels' cache mode
+    l.cached = fused ? 0 : cache_mode(g.nvol, mixed);
+    const char *cm = getenv("AWP_CACHED");
+    if (!fused && cm && cm[0] >= '0' && cm[0] <= '3' && !cm[1]) l.cached = cm[0] - '0';
     // Form and blocks per CU of the two-stage stress kernel, measured at
     // 1500x1000x300 with the tile patches and 25-level z chunks: the 32-bit
     // byte-offset form, as many blocks as registers allow, in both storage

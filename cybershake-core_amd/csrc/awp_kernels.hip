@@ -82,7 +82,7 @@ __device__ __forceinline__ void velocity_tile(const Geo &g, const State &s0, con
     for (int k = kb; k <= ke; ++k, o += sz) {
         const float xz_p1 = xz[o + sz];
         const float yz_p1 = yz[o + sz];
-        const float zz_p2 = nt_ld(&zz[o + 2 * sz]);   // zz: read at (i, j) only
+        const float zz_p2 = nt_ld<P::nt>(&zz[o + 2 * sz]);   // zz: read at (i, j) only
         const float db = P::mixed ? s.mbar[mbar_idx(g, 0, k)] : 0.0f;
         const float dA = mdec(d1[o], db), dB = mdec(d1[o - sy], db), dC = mdec(d1[o + 1], db),
                     dD = mdec(d1[o + 1 - sy], db);
@@ -93,7 +93,7 @@ __device__ __forceinline__ void velocity_tile(const Geo &g, const State &s0, con
         const float yy_0 = yy[o], yy_jp1 = yy[o + sy], yy_jp2 = yy[o + 2 * sy], yy_jm1 = yy[o - sy];
         const float xz_ip1 = xz[o + 1], xz_ip2 = xz[o + 2], xz_im1 = xz[o - 1];
         const float yz_jm1 = yz[o - sy], yz_jp1 = yz[o + sy], yz_jm2 = yz[o - 2 * sy];
-        float u0 = nt_ld(&s.u1[o]), v0 = nt_ld(&s.v1[o]), w0 = nt_ld(&s.w1[o]);
+        float u0 = nt_ld<P::nt>(&s.u1[o]), v0 = nt_ld<P::nt>(&s.v1[o]), w0 = nt_ld<P::nt>(&s.w1[o]);
         if (k == hook.k || k == hook.tk) hook_velocity(hook, i, j, k, dA, u0, v0, w0);
 
         float d, q, u, v, w;
@@ -116,9 +116,9 @@ __device__ __forceinline__ void velocity_tile(const Geo &g, const State &s0, con
             c1 * (yz_0 - yz_jm1) + c2 * (yz_jp1 - yz_jm2) +
             c1 * (zz_p1 - zz_0) + c2 * (zz_p2 - zz_m1));
         const float D = fxy * s.fz[k];
-        nt_st(&s.u1[o], u * D);
-        nt_st(&s.v1[o], v * D);
-        nt_st(&s.w1[o], w * D);
+        nt_st<P::nt>(&s.u1[o], u * D);
+        nt_st<P::nt>(&s.v1[o], v * D);
+        nt_st<P::nt>(&s.w1[o], w * D);
 
         xz_m2 = xz_m1; xz_m1 = xz_0; xz_0 = xz_p1;
         yz_m2 = yz_m1; yz_m1 = yz_0; yz_0 = yz_p1;
@@ -164,7 +164,7 @@ __device__ __forceinline__ void velocity_tile_b(const Geo &g, const State &s0, c
     for (int k = kb; k <= ke; ++k, p.up()) {
         const float xz_p1 = p.ld(xz, 0, 0, 1);
         const float yz_p1 = p.ld(yz, 0, 0, 1);
-        const float zz_p2 = gln(zz, p.at(0, 2));   // zz: read at (i, j) only
+        const float zz_p2 = gln<P::nt>(zz, p.at(0, 2));   // zz: read at (i, j) only
         const float db = P::mixed ? s.mbar[mbar_idx(g, 0, k)] : 0.0f;
         const float dA = mdec(p.ld(d1), db), dB = mdec(p.ld(d1, 0, -1), db), dC = mdec(p.ld(d1, 1), db),
                     dD = mdec(p.ld(d1, 1, -1), db);
@@ -175,7 +175,7 @@ __device__ __forceinline__ void velocity_tile_b(const Geo &g, const State &s0, c
         const float yy_0 = p.ld(yy), yy_jp1 = p.ld(yy, 0, 1), yy_jp2 = p.ld(yy, 0, 2), yy_jm1 = p.ld(yy, 0, -1);
         const float xz_ip1 = p.ld(xz, 1), xz_ip2 = p.ld(xz, 2), xz_im1 = p.ld(xz, -1);
         const float yz_jm1 = p.ld(yz, 0, -1), yz_jp1 = p.ld(yz, 0, 1), yz_jm2 = p.ld(yz, 0, -2);
-        float u0 = p.ldn(s.u1), v0 = p.ldn(s.v1), w0 = p.ldn(s.w1);
+        float u0 = p.template ldn<P::nt>(s.u1), v0 = p.template ldn<P::nt>(s.v1), w0 = p.template ldn<P::nt>(s.w1);
         if (k == hook.k || k == hook.tk) hook_velocity(hook, i, j, k, dA, u0, v0, w0);
 
         float d, q, u, v, w;
@@ -198,9 +198,9 @@ __device__ __forceinline__ void velocity_tile_b(const Geo &g, const State &s0, c
             c1 * (yz_0 - yz_jm1) + c2 * (yz_jp1 - yz_jm2) +
             c1 * (zz_p1 - zz_0) + c2 * (zz_p2 - zz_m1));
         const float D = fxy * s.fz[k];
-        p.stn(s.u1, u * D);
-        p.stn(s.v1, v * D);
-        p.stn(s.w1, w * D);
+        p.template stn<P::nt>(s.u1, u * D);
+        p.template stn<P::nt>(s.v1, v * D);
+        p.template stn<P::nt>(s.w1, w * D);
 
         xz_m2 = xz_m1; xz_m1 = xz_0; xz_0 = xz_p1;
         yz_m2 = yz_m1; yz_m1 = yz_0; yz_0 = yz_p1;
@@ -635,23 +635,23 @@ __device__ __forceinline__ void stress_tile_b(const Geo &g, const State &s0, con
         const float lb = P::mixed ? s.mbar[mbar_idx(g, 2, k)] : 0.0f;
         float lA, lB, lC, lD, mA, mB, mC, mD;
         if constexpr (P::mixed) {
-            const unsigned wA = p.ld(mlq), wB = p.ld(mlq, 1), wC = p.ld(mlq, 0, -1), wD = p.ld(mlq, 1, -1);
+            const unsigned wA = p.template ldm<P::ntm>(mlq), wB = p.template ldm<P::ntm>(mlq, 1), wC = p.template ldm<P::ntm>(mlq, 0, -1), wD = p.template ldm<P::ntm>(mlq, 1, -1);
             lA = mdec(h_hi(wA), lb); lB = mdec(h_hi(wB), lb); lC = mdec(h_hi(wC), lb); lD = mdec(h_hi(wD), lb);
             mA = mdec(h_lo(wA), mb); mB = mdec(h_lo(wB), mb); mC = mdec(h_lo(wC), mb); mD = mdec(h_lo(wD), mb);
         } else {
-            lA = mdec(p.ld(lam), lb); lB = mdec(p.ld(lam, 1), lb); lC = mdec(p.ld(lam, 0, -1), lb);
-            lD = mdec(p.ld(lam, 1, -1), lb);
-            mA = mdec(p.ld(mu), mb); mB = mdec(p.ld(mu, 1), mb); mC = mdec(p.ld(mu, 0, -1), mb);
-            mD = mdec(p.ld(mu, 1, -1), mb);
+            lA = mdec(p.template ldm<P::ntm>(lam), lb); lB = mdec(p.template ldm<P::ntm>(lam, 1), lb); lC = mdec(p.template ldm<P::ntm>(lam, 0, -1), lb);
+            lD = mdec(p.template ldm<P::ntm>(lam, 1, -1), lb);
+            mA = mdec(p.template ldm<P::ntm>(mu), mb); mB = mdec(p.template ldm<P::ntm>(mu, 1), mb); mC = mdec(p.template ldm<P::ntm>(mu, 0, -1), mb);
+            mD = mdec(p.template ldm<P::ntm>(mu, 1, -1), mb);
         }
         float pA, pB, pC, pD, sA, sB, sC, sD;
         if constexpr (P::mixed) {
-            const unsigned wA = p.ld(qq), wB = p.ld(qq, 1), wC = p.ld(qq, 0, -1), wD = p.ld(qq, 1, -1);
+            const unsigned wA = p.template ldm<P::ntm>(qq), wB = p.template ldm<P::ntm>(qq, 1), wC = p.template ldm<P::ntm>(qq, 0, -1), wD = p.template ldm<P::ntm>(qq, 1, -1);
             pA = q_lo(wA); pB = q_lo(wB); pC = q_lo(wC); pD = q_lo(wD);
             sA = q_hi(wA); sB = q_hi(wB); sC = q_hi(wC); sD = q_hi(wD);
         } else {
-            pA = ld(p.ld(qp)); pB = ld(p.ld(qp, 1)); pC = ld(p.ld(qp, 0, -1)); pD = ld(p.ld(qp, 1, -1));
-            sA = ld(p.ld(qs)); sB = ld(p.ld(qs, 1)); sC = ld(p.ld(qs, 0, -1)); sD = ld(p.ld(qs, 1, -1));
+            pA = ld(p.template ldm<P::ntm>(qp)); pB = ld(p.template ldm<P::ntm>(qp, 1)); pC = ld(p.template ldm<P::ntm>(qp, 0, -1)); pD = ld(p.template ldm<P::ntm>(qp, 1, -1));
+            sA = ld(p.template ldm<P::ntm>(qs)); sB = ld(p.template ldm<P::ntm>(qs, 1)); sC = ld(p.template ldm<P::ntm>(qs, 0, -1)); sD = ld(p.template ldm<P::ntm>(qs, 1, -1));
         }
 
         const float u_ip1 = p.ld(u1, 1), u_ip2 = p.ld(u1, 2), u_im1 = p.ld(u1, -1);
@@ -707,15 +707,15 @@ __device__ __forceinline__ void stress_tile_b(const Geo &g, const State &s0, con
         if constexpr (P::mixed) {
             // the exponents of this row segment: one 8-byte slot at byte offset xo
             ew = rexp_load(s.rexp, (long long)(xo >> 3));
-            r1 = r_decode(p.ldn(R1), rexp_of(ew, 0)); r2 = r_decode(p.ldn(R2), rexp_of(ew, 1));
-            r3 = r_decode(p.ldn(R3), rexp_of(ew, 2)); r4 = r_decode(p.ldn(R4), rexp_of(ew, 3));
-            r5 = r_decode(p.ldn(R5), rexp_of(ew, 4)); r6 = r_decode(p.ldn(R6), rexp_of(ew, 5));
+            r1 = r_decode(p.template ldn<P::ntr>(R1), rexp_of(ew, 0)); r2 = r_decode(p.template ldn<P::ntr>(R2), rexp_of(ew, 1));
+            r3 = r_decode(p.template ldn<P::ntr>(R3), rexp_of(ew, 2)); r4 = r_decode(p.template ldn<P::ntr>(R4), rexp_of(ew, 3));
+            r5 = r_decode(p.template ldn<P::ntr>(R5), rexp_of(ew, 4)); r6 = r_decode(p.template ldn<P::ntr>(R6), rexp_of(ew, 5));
         } else {
-            r1 = p.ldn(R1); r2 = p.ldn(R2); r3 = p.ldn(R3);
-            r4 = p.ldn(R4); r5 = p.ldn(R5); r6 = p.ldn(R6);
+            r1 = p.template ldn<P::ntr>(R1); r2 = p.template ldn<P::ntr>(R2); r3 = p.template ldn<P::ntr>(R3);
+            r4 = p.template ldn<P::ntr>(R4); r5 = p.template ldn<P::ntr>(R5); r6 = p.template ldn<P::ntr>(R6);
         }
-        float xx = p.ldn(s.xx), yy = p.ldn(s.yy), zz = p.ldn(s.zz);
-        float xy = p.ldn(s.xy), xz = p.ldn(s.xz), yz = p.ldn(s.yz);
+        float xx = p.template ldn<P::nt>(s.xx), yy = p.template ldn<P::nt>(s.yy), zz = p.template ldn<P::nt>(s.zz);
+        float xy = p.template ldn<P::nt>(s.xy), xz = p.template ldn<P::nt>(s.xz), yz = p.template ldn<P::nt>(s.yz);
 
         xx = xx + dth * (vtmp - 2.0f * vxm * (vt2 + vt3)) + dt * r1;
         yy = yy + dth * (vtmp - 2.0f * vxm * (vt1 + vt3)) + dt * r2;
@@ -763,14 +763,14 @@ __device__ __forceinline__ void stress_tile_b(const Geo &g, const State &s0, con
             const unsigned long long en = row_exponents6(rv, act, ew);
 #pragma unroll
             for (int q = 0; q < 6; ++q)
-                if (act) p.stn(RR[q], r_encode(rv[q], rexp_of(en, q)));
-            if (act && threadIdx.x == 0) gsn((G<unsigned long long> *)s.rexp, xo, en);
+                if (act) p.template stn<P::ntr>(RR[q], r_encode(rv[q], rexp_of(en, q)));
+            if (act && threadIdx.x == 0) gsn<P::nt>((G<unsigned long long> *)s.rexp, xo, en);
         } else {
-            p.stn(R1, r1); p.stn(R2, r2); p.stn(R3, r3);
-            p.stn(R4, r4); p.stn(R5, r5); p.stn(R6, r6);
+            p.template stn<P::ntr>(R1, r1); p.template stn<P::ntr>(R2, r2); p.template stn<P::ntr>(R3, r3);
+            p.template stn<P::ntr>(R4, r4); p.template stn<P::ntr>(R5, r5); p.template stn<P::ntr>(R6, r6);
         }
         if (act) {
-            p.stn(s.xx, xx); p.stn(s.yy, yy); p.stn(s.xy, xy);
+            p.template stn<P::nt>(s.xx, xx); p.template stn<P::nt>(s.yy, yy); p.template stn<P::nt>(s.xy, xy);
             if (k == g.nz) {
                 // fstr: images above the surface, xz = yz = 0 on it
                 p.st(s.zz, zz);
@@ -785,7 +785,7 @@ __device__ __forceinline__ void stress_tile_b(const Geo &g, const State &s0, con
                 hook_stress(hook, s, i, j, [&](const auto *a, int dk) { return p.ld(a, 0, 0, dk); },
                             [&](auto *a, float v, int dk) { p.st(a, v, 0, 0, dk); });
             } else {
-                p.stn(s.zz, zz); p.stn(s.xz, xz); p.stn(s.yz, yz);
+                p.template stn<P::nt>(s.zz, zz); p.template stn<P::nt>(s.xz, xz); p.template stn<P::nt>(s.yz, yz);
             }
         }
         xz_f2 = xz_f1; xz_f1 = xz;
@@ -1530,6 +1530,19 @@ static void str_batch_t(const Launch &l, const SJob *d_jobs, int njobs, int tota
                        dim3(TX, l.tile_y, l.tile_xw), l.lds_s, st, d_jobs, njobs, total, per, claim, l.xrot & 7, hook);
 }
 
+// the byte-offset stress kernel in the run's cache mode
+template <class P>
+static void cached_stress(const Launch &l, const SJob *d_jobs, int njobs, int total, int per, int grid_s,
+                          unsigned long long *claim, const Hook &hook, hipStream_t st)
+{
+    if (l.cached == 1)
+        str_batch_t<Cached<P, 0>, 1, true, 512>(l, d_jobs, njobs, total, per, grid_s, claim, hook, st);
+    else if (l.cached == 2)
+        str_batch_t<Cached<P, 1>, 1, true, 512>(l, d_jobs, njobs, total, per, grid_s, claim, hook, st);
+    else
+        str_batch_t<Cached<P, 2>, 1, true, 512>(l, d_jobs, njobs, total, per, grid_s, claim, hook, st);
+}
+
 template <class P>
 static hipError_t stress_stage(const Launch &l, bool os, const SJob *d_jobs, int njobs, int total, int per,
                                int grid_s, unsigned long long *claim, const Hook &hook, hipStream_t st)
@@ -1555,6 +1568,11 @@ hipError_t launch_split_velocity(bool mixed, const Launch &l, bool o32, const SJ
     if (njobs <= 0 || total <= 0) return hipSuccess;
     const int per = (total + 7) / 8;
     const bool ov = o32 && l.o32_v;
+    if (l.cached && l.unroll != 2 && !tall(l)) {
+        if (mixed) vel_batch_t<Cached<StoreMixed, 0>, 1, 512>(l, ov, d_jobs, njobs, total, per, grid_v, claim, hook, st);
+        else vel_batch_t<Cached<StoreF32, 0>, 1, 512>(l, ov, d_jobs, njobs, total, per, grid_v, claim, hook, st);
+        return hipGetLastError();
+    }
     const hipError_t e = mixed ? velocity_stage<StoreMixed>(l, ov, d_jobs, njobs, total, per, grid_v, claim, hook, st)
                                : velocity_stage<StoreF32>(l, ov, d_jobs, njobs, total, per, grid_v, claim, hook, st);
     if (e != hipSuccess) return e;
@@ -1567,6 +1585,11 @@ hipError_t launch_split_stress(bool mixed, const Launch &l, bool o32, const SJob
     if (njobs <= 0 || total <= 0) return hipSuccess;
     const int per = (total + 7) / 8;
     const bool os = o32 && l.o32_s;
+    if (l.cached && os && l.unroll != 2 && !tall(l)) {
+        if (mixed) cached_stress<StoreMixed>(l, d_jobs, njobs, total, per, grid_s, claim, hook, st);
+        else cached_stress<StoreF32>(l, d_jobs, njobs, total, per, grid_s, claim, hook, st);
+        return hipGetLastError();
+    }
     const hipError_t e = mixed ? stress_stage<StoreMixed>(l, os, d_jobs, njobs, total, per, grid_s, claim, hook, st)
                                : stress_stage<StoreF32>(l, os, d_jobs, njobs, total, per, grid_s, claim, hook, st);
     if (e != hipSuccess) return e;

@@ -81,6 +81,12 @@ __device__ inline unsigned long long rexp_pack(const int e[6])
     return w;
 }
 
+// the non-temporal hint on pointwise accesses; AWP_NT=0 at compile time turns
+// it off everywhere
+#ifndef AWP_NT
+#define AWP_NT 1
+#endif
+
 // ---- storage element types ------------------------------------------------
 struct Bf16 {
     unsigned short u;
@@ -108,12 +114,22 @@ struct StoreF32 {
     using Q = float;   // qp, qs
     using M = float;   // d1, mu, lam
     static constexpr bool mixed = false;
+    // the non-temporal hint (nt_ld) on pointwise wavefields, on r1..r6 and on
+    // the stress kernel's media
+    static constexpr bool nt = AWP_NT != 0, ntr = AWP_NT != 0, ntm = false;
 };
 struct StoreMixed {
     using R = _Float16;   // r * 2^(15-e), e per row segment (see below)
     using Q = _Float16;
     using M = _Float16;   // x / b(k) - 1, b(k) the level's profile value
     static constexpr bool mixed = true;
+    static constexpr bool nt = AWP_NT != 0, ntr = AWP_NT != 0, ntm = false;
+};
+// the same storage with the wavefields cached; STREAM 1: r1..r6 streamed, 2:
+// the media of the stress kernel too (cache_mode)
+template <class P, int STREAM>
+struct Cached : P {
+    static constexpr bool nt = false, ntr = AWP_NT != 0 && STREAM >= 1, ntm = AWP_NT != 0 && STREAM >= 2;
 };
 
 // The density and the compliances from their storage: FP32 as stored, or
@@ -321,37 +337,34 @@ __device__ __forceinline__ void gs(G<T> *base, O off, T v, int imm = 0)
 }
 // Streamed access.  A value of a pointwise array (one read and one write per
 // step at the point itself, never a neighbour's halo) goes through the
-// caches with the non-temporal hint, leaving L2 to the halo lines of the
-// stencil arrays that neighbouring tiles read again.  AWP_NT=0 at compile
-// time turns the hint off.
-#ifndef AWP_NT
-#define AWP_NT 1
-#endif
-template <class T>
+// caches with the non-temporal hint (NT), leaving L2 to the halo lines of the
+// stencil arrays that neighbouring tiles read again -- unless the run's
+// wavefields can stay in the memory-side cache (cache_mode).
+template <bool NT, class T>
 __device__ __forceinline__ T nt_ld(const G<T> *a)
 {
-    if constexpr (AWP_NT != 0)
+    if constexpr (NT)
         return __builtin_nontemporal_load(a);
     else
         return *a;
 }
-template <class T>
+template <bool NT, class T>
 __device__ __forceinline__ void nt_st(G<T> *a, T v)
 {
-    if constexpr (AWP_NT != 0)
+    if constexpr (NT)
         __builtin_nontemporal_store(v, a);
     else
         *a = v;
 }
-template <class T, class O>
-__device__ __forceinline__ T gln(const G<T> *base, O off)
+template <bool NT = AWP_NT != 0, class T, class O>
+__device__ __forceinline__ T gln(const G<T> *base, O off, int imm = 0)
 {
-    return nt_ld(reinterpret_cast<const G<T> *>(reinterpret_cast<const G<char> *>(base) + off));
+    return nt_ld<NT>(reinterpret_cast<const G<T> *>(reinterpret_cast<const G<char> *>(base) + off + imm));
 }
-template <class T, class O>
+template <bool NT = AWP_NT != 0, class T, class O>
 __device__ __forceinline__ void gsn(G<T> *base, O off, T v)
 {
-    nt_st(reinterpret_cast<G<T> *>(reinterpret_cast<G<char> *>(base) + off), v);
+    nt_st<NT>(reinterpret_cast<G<T> *>(reinterpret_cast<G<char> *>(base) + off), v);
 }
 // Position of one thread's point in the volume arrays while it marches up in
 // z, as a 32-bit byte offset into a 4-byte array (2-byte arrays take it
@@ -375,16 +388,22 @@ struct Cursor32 {
     {
         gs(p, at(dj, dk) >> (sizeof(T) == 2 ? 1 : 0), v, di * (int)sizeof(T));
     }
+    // ld with the hint
+    template <bool NT, class T>
+    __device__ __forceinline__ T ldm(const G<T> *p, int di = 0, int dj = 0) const
+    {
+        return gln<NT>(p, at(dj, 0) >> (sizeof(T) == 2 ? 1 : 0), di * (int)sizeof(T));
+    }
     // the point itself, streamed (nt_ld / nt_st)
-    template <class T>
+    template <bool NT, class T>
     __device__ __forceinline__ T ldn(const G<T> *p) const
     {
-        return gln(p, o >> (sizeof(T) == 2 ? 1 : 0));
+        return gln<NT>(p, o >> (sizeof(T) == 2 ? 1 : 0));
     }
-    template <class T>
+    template <bool NT, class T>
     __device__ __forceinline__ void stn(G<T> *p, T v) const
     {
-        gsn(p, o >> (sizeof(T) == 2 ? 1 : 0), v);
+        gsn<NT>(p, o >> (sizeof(T) == 2 ? 1 : 0), v);
     }
     __device__ __forceinline__ void up() { o += sz; }
 };
@@ -417,6 +436,27 @@ static inline int split_nchunk(int nz, int kc)
 {
     const int n = (nz + kc / 2) / kc;
     return n < 1 ? 1 : n;
+}
+
+// What of nvol points' step arrays the two-stage kernels keep in the 256 MB
+// memory-side cache from step to step, by what fits it (bytes a point, FP32 /
+// mixed): 1 everything (80 / 52), 2 all but r1..r6 (56 / 46), which stream
+// past it with the non-temporal hint, 3 the wavefields and d1 (40 / 38); 0
+// nothing: every pointwise access streams, which from there on is the faster.
+// Streams in the stress kernel's mix run at 7.7 TB/s from that cache, 6.1
+// with the hint, 5.0 from HBM.  Microseconds per step in mode 0 / 1 / 2 / 3,
+// FP32: 150x150x90 (2.8M points with padding) 108 / 80 / 97 / --; 180x160x90
+// (3.9M) 125 / 127 / 111 / 118; 203x187x101 (5.1M) 183 / 188 / 174 / 169;
+// 240x220x80 (6.0M) 181 / 189 / 177 / 171; 260x220x100 (7.5M) 268 / 285 / 271
+// / 268; 250x250x110 (9.3M) 281 / 296 / 285 / 287.  Mixed: 180x160x90 115 /
+// 89 / 101 / 105; 203x187x101 167 / 162 / 149 / 153; 240x220x80 163 / 165 /
+// 145 / 151; 260x220x100 231 / 242 / 233 / 226; 250x250x110 239 / 250 / 245 /
+// 245.
+static inline int cache_mode(long long nvol, bool mixed)
+{
+    if (nvol * (mixed ? 52 : 80) <= 250000000ll) return 1;
+    if (nvol * (mixed ? 46 : 56) <= 280000000ll) return 2;
+    return nvol * (mixed ? 38 : 40) <= 285000000ll ? 3 : 0;
 }
 
 // The fused step addresses every volume array with 32-bit byte offsets
@@ -462,6 +502,7 @@ struct Launch {
     int spw, sph;    // two-stage kernels: tile patch width / height (0 = rows of tiles)
     bool o32;        // 32-bit byte offsets reach every array (offsets32() of the run's geometry)
     bool o32_s;      // two-stage stress kernel: its 32-bit byte-offset form (only where o32)
+    int cached;      // two-stage kernels: cache_mode() of the run
     bool o32_v;      // two-stage velocity kernel: its 32-bit byte-offset form (only where o32)
     int bpc_v, bpc_s;   // two-stage kernels: most blocks per CU (0 = as registers allow)
     unsigned lds_v, lds_s;   // the dynamic LDS bytes per block that enforce them (set_block_caps)
