@@ -13,10 +13,12 @@
 #include <unistd.h>
 
 #include <algorithm>
+#include <atomic>
 #include <mutex>
 #include <string>
 #include <vector>
 
+#include "../host/awp_par.h"
 #include "awp_ctx.hpp"
 #include "awp_kernels.hpp"
 #include "awpsgt.h"
@@ -372,6 +374,9 @@ extern "C" int awp_create(awp_ctx **out, const awp_in3d *p, int device, int stor
     ctx->sg_done = false;
     ctx->d_trace = nullptr;
     ctx->trace_pos = 0;
+    ctx->pin = nullptr;
+    ctx->pin_half = 0;
+    ctx->pin_ev[0] = ctx->pin_ev[1] = nullptr;
 
     e = hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking);
     if (e != hipSuccess) {
@@ -500,6 +505,9 @@ extern "C" int awp_destroy(awp_ctx *ctx)
     hipFree(ctx->d_kidx);
     hipFree(ctx->d_sg);
     hipFree(ctx->d_sgt);
+    if (ctx->pin) hipHostFree(ctx->pin);
+    for (hipEvent_t ev : ctx->pin_ev)
+        if (ev) hipEventDestroy(ev);
     if (ctx->stream) hipStreamDestroy(ctx->stream);
     delete ctx;
     return AWP_OK;
@@ -1250,6 +1258,96 @@ extern "C" int awp_device_bytes(const awp_ctx *ctx, size_t *bytes)
 // ---------------------------------------------------------------------------
 // outputs
 // ---------------------------------------------------------------------------
+namespace {
+
+// Moves `bytes` of device memory through the run's pinned staging buffer in
+// order, in pieces of whole units (the last may be shorter): make(half, off,
+// n, &src) enqueues on the run's stream what produces bytes [off, off + n) and
+// says where they are, use(host, off, n) takes them on the host while the next
+// piece is on its way.  (A pageable copy runs at 10-17 GB/s through the
+// runtime's own staging, a pinned one at 57.)
+constexpr size_t PIN_HALF = (size_t)16 << 20;
+
+int drain_room(awp_ctx *ctx, size_t unit)
+{
+    const size_t half = std::max(PIN_HALF, unit);
+    for (int k = 0; k < 2; ++k)
+        if (!ctx->pin_ev[k]) HIPTRY(ctx, hipEventCreateWithFlags(&ctx->pin_ev[k], hipEventDisableTiming));
+    if (ctx->pin_half >= half) return AWP_OK;
+    if (ctx->pin) hipHostFree(ctx->pin);
+    ctx->pin = nullptr;
+    ctx->pin_half = 0;
+    const hipError_t e = hipHostMalloc((void **)&ctx->pin, 2 * half, hipHostMallocDefault);
+    if (e != hipSuccess) {
+        ctx->pin = nullptr;
+        return fail(ctx, AWP_ENOMEM, "hipHostMalloc(%zu): %s", 2 * half, hipGetErrorString(e));
+    }
+    ctx->pin_half = half;
+    return AWP_OK;
+}
+
+template <class MAKE, class USE>
+int drain(awp_ctx *ctx, size_t bytes, size_t unit, MAKE make, USE use)
+{
+    if (!bytes) return AWP_OK;
+    const int room = drain_room(ctx, unit);
+    if (room) return room;
+    const size_t half = ctx->pin_half, step = half / unit * unit;
+    size_t sent = 0, done = 0;
+    for (int k = 0; done < bytes; k ^= 1) {
+        // keep one piece on its way beside the one in use
+        while (sent < bytes && sent < done + 2 * step) {
+            const int h = (int)(sent / step & 1);
+            const size_t n = std::min(step, bytes - sent);
+            const void *src = nullptr;
+            int rc = make(h, sent, n, &src);
+            if (rc) return rc;
+            HIPTRY(ctx, hipMemcpyAsync(ctx->pin + h * half, src, n, hipMemcpyDeviceToHost, ctx->stream));
+            HIPTRY(ctx, hipEventRecord(ctx->pin_ev[h], ctx->stream));
+            sent += n;
+        }
+        const size_t n = std::min(step, bytes - done);
+        HIPTRY(ctx, hipEventSynchronize(ctx->pin_ev[k]));
+        int rc = use(ctx->pin + k * half, done, n);
+        if (rc) {
+            hipStreamSynchronize(ctx->stream);   // the piece on its way still lands in the buffer
+            return rc;
+        }
+        done += n;
+    }
+    return AWP_OK;
+}
+
+// fn(a, b) over parts [a, b) of n items, on as many threads as `bytes` of
+// copying are worth
+template <class FN>
+void parts(size_t n, size_t bytes, FN fn)
+{
+    struct Arg {
+        size_t n;
+        FN *fn;
+    } arg = {n, &fn};
+    const int np = (int)std::min<size_t>(awp_par_threads(bytes), std::max<size_t>(n, 1));
+    awp_par(np, [](void *p, int k, int m) {
+        Arg *a = (Arg *)p;
+        (*a->fn)(a->n * (size_t)k / (size_t)m, a->n * (size_t)(k + 1) / (size_t)m);
+    }, &arg);
+}
+
+bool write_at(int fd, const char *p, size_t n, off_t off)
+{
+    while (n) {
+        const ssize_t w = pwrite(fd, p, n, off);
+        if (w <= 0) return false;
+        p += w;
+        off += w;
+        n -= (size_t)w;
+    }
+    return true;
+}
+
+}  // namespace
+
 extern "C" int awp_get_sgt(awp_ctx *ctx, float *host, size_t count)
 {
     if (!ctx || !host) return AWP_EINVAL;
@@ -1257,9 +1355,20 @@ extern "C" int awp_get_sgt(awp_ctx *ctx, float *host, size_t count)
     const size_t n = (size_t)ctx->npts * 6 * ctx->nsamp_max;
     if (count < n) return fail(ctx, AWP_EINVAL, "buffer holds %zu floats, need %zu", count, n);
     HIPTRY(ctx, hipSetDevice(ctx->device));
-    HIPTRY(ctx, hipStreamSynchronize(ctx->stream));
-    if (n) HIPTRY(ctx, hipMemcpy(host, ctx->d_sgt, n * sizeof(float), hipMemcpyDeviceToHost));
-    return AWP_OK;
+    if (n * sizeof(float) < ((size_t)8 << 20)) {
+        HIPTRY(ctx, hipStreamSynchronize(ctx->stream));
+        if (n) HIPTRY(ctx, hipMemcpy(host, ctx->d_sgt, n * sizeof(float), hipMemcpyDeviceToHost));
+        return AWP_OK;
+    }
+    return drain(ctx, n * sizeof(float), 64,
+                 [ctx](int, size_t off, size_t, const void **src) {
+                     *src = (const char *)ctx->d_sgt + off;
+                     return AWP_OK;
+                 },
+                 [host](const char *p, size_t off, size_t m) {
+                     parts(m, m, [=](size_t a, size_t b) { memcpy((char *)host + off + a, p + a, b - a); });
+                     return AWP_OK;
+                 });
 }
 
 extern "C" int awp_get_trace(awp_ctx *ctx, float *host, size_t count, int *ijk)
@@ -1288,52 +1397,51 @@ extern "C" int awp_write_sgt_file(awp_ctx *ctx, const char *path)
     const int avail = std::min(nflush, ctx->nsamp / p.write_step);
     if (avail <= 0) return AWP_OK;   // the reference opens the file at the first flush
     const int ws = p.write_step, ms = ctx->nsamp_max;
-    const size_t pts_per_chunk = 16384;
-    std::vector<float> host(pts_per_chunk * 6 * (size_t)ms);
     int fd = open(path, O_WRONLY | O_CREAT | O_TRUNC, 0644);
     if (fd < 0) return fail(ctx, AWP_EIO, "cannot create '%s'", path);
-    HIPTRY(ctx, hipSetDevice(ctx->device));
-    HIPTRY(ctx, hipStreamSynchronize(ctx->stream));
+    hipError_t e = hipSetDevice(ctx->device);
     const size_t slot = (size_t)4 * nt_out;          // bytes per (point, component)
-    std::vector<char> img;
-    for (size_t g0 = 0; g0 < (size_t)ctx->npts; g0 += pts_per_chunk) {
-        const size_t g1 = std::min((size_t)ctx->npts, g0 + pts_per_chunk);
-        size_t last = g1;   // one past the last kept point of the chunk
-        while (last > g0 && !ctx->keep[last - 1]) --last;
-        size_t first = g0;
-        while (first < last && !ctx->keep[first]) ++first;
-        if (first >= last) continue;
-        const size_t n = (size_t)(last - g0) * 6 * ms;
-        hipError_t e = hipMemcpy(host.data(), ctx->d_sgt + g0 * 6 * (size_t)ms, n * sizeof(float), hipMemcpyDeviceToHost);
-        if (e != hipSuccess) {
-            close(fd);
-            return fail(ctx, AWP_EHIP, "hipMemcpy SGT: %s", hipGetErrorString(e));
+    const size_t rec = (size_t)6 * ms * sizeof(float);   // a point in HBM
+    std::atomic<bool> ok(true);
+    // points [g0 + a, g0 + b) from their series at p: the file bytes from the
+    // first kept point to the last one's last full buffer (a dropped point
+    // beyond them stays a hole)
+    auto put = [&](const char *src, size_t g0, size_t a, size_t b) {
+        while (b > a && !ctx->keep[g0 + b - 1]) --b;
+        while (a < b && !ctx->keep[g0 + a]) ++a;
+        if (a >= b) return;
+        const size_t off0 = (g0 + a) * 6 * slot;
+        const size_t end = (g0 + b - 1) * 6 * slot + 5 * slot + (size_t)avail * 4 * ws;
+        char *img = (char *)calloc(1, end - off0);
+        if (!img) {
+            ok = false;
+            return;
         }
-        // image of the file bytes [first*24*nt_out, end of last point's last flush)
-        const size_t off0 = first * 6 * slot;
-        const size_t end = (last - 1) * 6 * slot + 5 * slot + (size_t)(avail - 1) * 4 * ws + 4 * (size_t)ws;
-        img.assign(end - off0, 0);
-        for (size_t g = first; g < last; ++g) {
-            if (!ctx->keep[g]) continue;
+        for (size_t g = a; g < b; ++g) {
+            if (!ctx->keep[g0 + g]) continue;
             for (int c = 0; c < 6; ++c)
-                for (int f = 1; f <= avail; ++f) {
-                    const size_t off = g * 6 * slot + c * slot + (size_t)(f - 1) * 4 * ws;
-                    memcpy(&img[off - off0], &host[((g - g0) * 6 + c) * (size_t)ms + (size_t)(f - 1) * ws],
-                           4 * (size_t)ws);
-                }
+                memcpy(img + ((g0 + g) * 6 + c) * slot - off0, src + g * rec + (size_t)c * ms * sizeof(float),
+                       (size_t)avail * 4 * ws);
         }
-        size_t done = 0;
-        while (done < img.size()) {
-            ssize_t w = pwrite(fd, img.data() + done, img.size() - done, (off_t)(off0 + done));
-            if (w <= 0) {
-                close(fd);
-                return fail(ctx, AWP_EIO, "write '%s' failed", path);
-            }
-            done += (size_t)w;
-        }
+        if (!write_at(fd, img, end - off0, (off_t)off0)) ok = false;
+        free(img);
+    };
+    int rc = AWP_OK;
+    if (e != hipSuccess) {
+        rc = fail(ctx, AWP_EHIP, "hipSetDevice: %s", hipGetErrorString(e));
+    } else {
+        rc = drain(ctx, (size_t)ctx->npts * rec, rec,
+                   [ctx](int, size_t off, size_t, const void **src) {
+                       *src = (const char *)ctx->d_sgt + off;
+                       return AWP_OK;
+                   },
+                   [&](const char *h, size_t off, size_t m) {
+                       parts(m / rec, 2 * m, [&](size_t a, size_t b) { put(h, off / rec, a, b); });
+                       return ok ? AWP_OK : fail(ctx, AWP_EIO, "write '%s' failed", path);
+                   });
     }
-    if (close(fd)) return fail(ctx, AWP_EIO, "close '%s' failed", path);
-    return AWP_OK;
+    if (close(fd) && rc == AWP_OK) return fail(ctx, AWP_EIO, "close '%s' failed", path);
+    return rc;
 }
 
 extern "C" int awp_write_sgt_file_rwg(awp_ctx *ctx, const char *path, int zsource)
@@ -1357,35 +1465,40 @@ extern "C" int awp_write_sgt_file_rwg(awp_ctx *ctx, const char *path, int zsourc
     const size_t raw_size = last < 0 ? 0 : (size_t)last * 6 * slot + 5 * slot + (size_t)avail * 4 * p.write_step;
     const size_t nrec = raw_size / (6 * slot);
     const int navail = avail * p.write_step;
-    FILE *f = fopen(path, "wb");
-    if (!f) return fail(ctx, AWP_EIO, "cannot create '%s'", path);
-    HIPTRY(ctx, hipSetDevice(ctx->device));
-    HIPTRY(ctx, hipStreamSynchronize(ctx->stream));
-    const size_t chunk = 8192;
-    const size_t per = 6 * (size_t)nt_out;
+    int fd = open(path, O_WRONLY | O_CREAT | O_TRUNC, 0666);
+    if (fd < 0) return fail(ctx, AWP_EIO, "cannot create '%s'", path);
+    const size_t unit = 6 * slot;   // a record of the file
     float *d_out = nullptr;
     int *d_keep = nullptr;
-    std::vector<float> host(chunk * per);
-    std::vector<int> kk(chunk);
-    hipError_t e = hipMalloc((void **)&d_out, std::max<size_t>(chunk * per, 1) * sizeof(float));
-    if (e == hipSuccess) e = hipMalloc((void **)&d_keep, chunk * sizeof(int));
-    bool ok = e == hipSuccess;
-    for (size_t g0 = 0; ok && g0 < nrec; g0 += chunk) {
-        const size_t n = std::min(chunk, nrec - g0);
-        for (size_t k = 0; k < n; ++k) kk[k] = ctx->keep[g0 + k];
-        e = hipMemcpy(d_keep, kk.data(), n * sizeof(int), hipMemcpyHostToDevice);
-        if (e == hipSuccess)
-            e = launch_sgt_rwg(ctx->d_sgt, d_keep, (int)g0, (int)n, ctx->nsamp_max, nt_out, navail, zsource ? 1 : 0,
-                               d_out, ctx->stream);
-        if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
-        if (e == hipSuccess) e = hipMemcpy(host.data(), d_out, n * per * sizeof(float), hipMemcpyDeviceToHost);
-        ok = e == hipSuccess && fwrite(host.data(), sizeof(float), n * per, f) == n * per;
-    }
+    hipError_t e = hipSetDevice(ctx->device);
+    int rc = e == hipSuccess ? drain_room(ctx, unit) : AWP_OK;
+    if (rc == AWP_OK && e == hipSuccess) e = hipMalloc((void **)&d_out, 2 * ctx->pin_half);
+    if (rc == AWP_OK && e == hipSuccess) e = hipMalloc((void **)&d_keep, std::max<size_t>(nrec, 1) * sizeof(int));
+    if (rc == AWP_OK && e == hipSuccess && nrec)
+        e = hipMemcpy(d_keep, ctx->keep.data(), nrec * sizeof(int), hipMemcpyHostToDevice);
+    if (rc == AWP_OK && e == hipSuccess)
+        rc = drain(ctx, nrec * unit, unit,
+                   [&](int h, size_t off, size_t n, const void **src) -> int {
+                       float *out = (float *)((char *)d_out + (size_t)h * ctx->pin_half);
+                       *src = out;
+                       const size_t g0 = off / unit;
+                       HIPTRY(ctx, launch_sgt_rwg(ctx->d_sgt, d_keep + g0, (int)g0, (int)(n / unit), ctx->nsamp_max,
+                                                  nt_out, navail, zsource ? 1 : 0, out, ctx->stream));
+                       return AWP_OK;
+                   },
+                   [&](const char *h, size_t off, size_t m) {
+                       std::atomic<bool> ok(true);
+                       parts(m / unit, m, [&](size_t a, size_t b) {
+                           if (!write_at(fd, h + a * unit, (b - a) * unit, (off_t)(off + a * unit))) ok = false;
+                       });
+                       return ok ? AWP_OK : fail(ctx, AWP_EIO, "write '%s' failed", path);
+                   });
     hipFree(d_out);
     hipFree(d_keep);
-    ok = (fclose(f) == 0) && ok;
+    const bool closed = close(fd) == 0;
     if (e != hipSuccess) return fail(ctx, AWP_EHIP, "RWG SGT: %s", hipGetErrorString(e));
-    return ok ? AWP_OK : fail(ctx, AWP_EIO, "write '%s' failed", path);
+    if (rc) return rc;
+    return closed ? AWP_OK : fail(ctx, AWP_EIO, "write '%s' failed", path);
 }
 
 extern "C" int awp_write_sgt_file_fp16(awp_ctx *ctx, const char *path)
@@ -1412,15 +1525,12 @@ extern "C" int awp_write_sgt_file_fp16(awp_ctx *ctx, const char *path)
     if (e == hipSuccess) e = hipMemsetAsync(d_data, 0, ndata * sizeof(_Float16), ctx->stream);
     if (e == hipSuccess && nsamp > 0)
         e = launch_sgt_fp16(ctx->d_sgt, ctx->d_kidx, ctx->nkept, ctx->nsamp_max, nsamp, d_scale, d_data, ctx->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
-    std::vector<float> scale(npts * 6);
-    std::vector<uint16_t> data(npts * 6 * (size_t)nsamp);
-    if (e == hipSuccess && npts) e = hipMemcpy(scale.data(), d_scale, npts * 6 * sizeof(float), hipMemcpyDeviceToHost);
-    if (e == hipSuccess && !data.empty())
-        e = hipMemcpy(data.data(), d_data, data.size() * sizeof(uint16_t), hipMemcpyDeviceToHost);
-    hipFree(d_scale);
-    hipFree(d_data);
-    if (e != hipSuccess) return fail(ctx, AWP_EHIP, "FP16 SGT: %s", hipGetErrorString(e));
+    if (e != hipSuccess) {
+        hipStreamSynchronize(ctx->stream);
+        hipFree(d_scale);
+        hipFree(d_data);
+        return fail(ctx, AWP_EHIP, "FP16 SGT: %s", hipGetErrorString(e));
+    }
     unsigned char hdr[64];
     memset(hdr, 0, sizeof(hdr));
     memcpy(hdr, "AWPSGT16", 8);
@@ -1431,13 +1541,35 @@ extern "C" int awp_write_sgt_file_fp16(awp_ctx *ctx, const char *path)
     memcpy(hdr + 28, &p.dt, 4);
     const uint32_t nto = (uint32_t)nt_out;   // the raw file's series length
     memcpy(hdr + 32, &nto, 4);
-    FILE *f = fopen(path, "wb");
-    if (!f) return fail(ctx, AWP_EIO, "cannot create '%s'", path);
-    bool ok = fwrite(hdr, 1, 64, f) == 64;
-    ok = ok && fwrite(scale.data(), sizeof(float), scale.size(), f) == scale.size();
-    ok = ok && fwrite(data.data(), sizeof(uint16_t), data.size(), f) == data.size();
-    ok = (fclose(f) == 0) && ok;
-    return ok ? AWP_OK : fail(ctx, AWP_EIO, "write '%s' failed", path);
+    int fd = open(path, O_WRONLY | O_CREAT | O_TRUNC, 0666);
+    int rc = fd < 0 ? fail(ctx, AWP_EIO, "cannot create '%s'", path)
+                    : write_at(fd, (const char *)hdr, 64, 0) ? AWP_OK : fail(ctx, AWP_EIO, "write '%s' failed", path);
+    // the header, then the scales, then the series
+    size_t base = 64;
+    const struct {
+        const void *dev;
+        size_t bytes;
+    } piece[2] = {{d_scale, npts * 6 * sizeof(float)}, {d_data, npts * 6 * (size_t)nsamp * sizeof(uint16_t)}};
+    for (int q = 0; q < 2 && rc == AWP_OK; ++q) {
+        rc = drain(ctx, piece[q].bytes, 64,
+                   [&](int, size_t off, size_t, const void **src) {
+                       *src = (const char *)piece[q].dev + off;
+                       return AWP_OK;
+                   },
+                   [&](const char *h, size_t off, size_t m) {
+                       std::atomic<bool> ok(true);
+                       parts(m, m, [&](size_t a, size_t b) {
+                           if (!write_at(fd, h + a, b - a, (off_t)(base + off + a))) ok = false;
+                       });
+                       return ok ? AWP_OK : fail(ctx, AWP_EIO, "write '%s' failed", path);
+                   });
+        base += piece[q].bytes;
+    }
+    hipStreamSynchronize(ctx->stream);
+    hipFree(d_scale);
+    hipFree(d_data);
+    if (fd >= 0 && close(fd) && rc == AWP_OK) rc = fail(ctx, AWP_EIO, "write '%s' failed", path);
+    return rc;
 }
 
 extern "C" int awp_get_field(awp_ctx *ctx, int which, int kext, float *host)

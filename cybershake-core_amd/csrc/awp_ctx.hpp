@@ -67,6 +67,11 @@ struct awp_ctx {
     float *d_sg;
     float *d_sgt;            // [npts][6][nsamp_max]
     std::vector<int> keep;   // per cordfile point
+    // pinned staging of the SGT output (drain): two halves of pin_half bytes,
+    // made on the first large read and kept for the next
+    char *pin;
+    size_t pin_half;
+    hipEvent_t pin_ev[2];
     // progress
     bool media_set, source_set, points_set, initialised;
     int step, nsamp;
