@@ -841,18 +841,20 @@ __device__ inline const SJob &split_tile(const SJob *__restrict__ jobs, const in
 // XCD's contiguous range of the global tile list with stride gridDim.x / 8
 // (k: the block's tiles so far), so the blocks of one XCD work on
 // neighbouring tiles of one run at a time and read each other's halo lines
-// from that XCD's L2.  `next`: the block's LDS broadcast slot.
+// from that XCD's L2; bit 3 of `rot` walks the ranges backwards.  `next`: the
+// block's LDS broadcast slot.
 __device__ inline int stage_tile(unsigned long long *claim, int per, int total, int rot, int k, int *next)
 {
     if (claim) {
         __syncthreads();   // every thread has read the previous tile
-        if (threadIdx.x == 0 && threadIdx.y == 0 && threadIdx.z == 0) *next = claim_tile(claim, per, total, rot);
+        if (threadIdx.x == 0 && threadIdx.y == 0 && threadIdx.z == 0) *next = claim_tile(claim, per, total, rot & 7);
         __syncthreads();
         return *next;
     }
     const int xcd = blockIdx.x & 7, slot = (int)(blockIdx.x >> 3) + k * (int)(gridDim.x >> 3);
-    const int tile = xcd * per + slot;
-    return (slot < per && tile < total) ? tile : -1;
+    const int n = min(per, total - xcd * per);   // tiles of the range
+    if (slot >= n) return -1;
+    return xcd * per + ((rot & 8) ? n - 1 - slot : slot);
 }
 
 // Persistent stage kernels over the job table (stage_tile assigns tiles).
@@ -1522,12 +1524,20 @@ static hipError_t velocity_stage(const Launch &l, bool ov, const SJob *d_jobs, i
     return hipSuccess;
 }
 
+// Beyond the cache modes the stress kernel walks the tiles the other way
+// round, so that it starts on what the velocity kernel touched last and the
+// next velocity kernel on what it touched last itself: 256 MB of each pass
+// come from the memory-side cache.  us per step, FP32 / mixed, against the
+// same way round: 300x300x120 476 -> 462 / 400 -> 390, 400x300x150 743 -> 723 /
+// 630 -> 612, 517x389x149 1248 -> 1223 / 1049 -> 1026, 800x600x200 3621 -> 3598
+// / 2987 -> 2961, 1500x1000x300 17264 -> 17209 / 14284 -> 14181; a run within
+// a cache mode loses by it (200x200x100 183 -> 185, 158 -> 159).
 template <class P, int U, bool O32, int MAXT>
 static void str_batch_t(const Launch &l, const SJob *d_jobs, int njobs, int total, int per, int grid_s,
                         unsigned long long *claim, const Hook &hook, hipStream_t st)
 {
     hipLaunchKernelGGL((k_stress_batch<P, U, O32, MAXT>), dim3(persistent_grid(grid_s, per, total, claim)),
-                       dim3(TX, l.tile_y, l.tile_xw), l.lds_s, st, d_jobs, njobs, total, per, claim, l.xrot & 7, hook);
+                       dim3(TX, l.tile_y, l.tile_xw), l.lds_s, st, d_jobs, njobs, total, per, claim, l.xrot & 7 | (l.cached == 0 ? 8 : 0), hook);
 }
 
 // the byte-offset stress kernel in the run's cache mode
