@@ -323,6 +323,12 @@ extern "C" int awp_batch_create(awp_batch **out, awp_ctx *const *runs, int nruns
         long long nvol = 0;
         for (int r = 0; r < nruns; ++r) nvol += runs[r]->g.nvol;
         if (b->split && nruns > 1) b->l.cached = cache_mode(nvol, b->mixed);
+        b->l.o32 = b->o32;
+        if (runs[0]->fused) b->l.claim = 0;   // a fused run's claims
+        if (b->split && !b->persist)
+            choose_staged(b->l, b->mixed);
+        else
+            b->l.staged = false;
     }
     b->nchunk.assign(nruns, 1);
     // the chain of a wave's levels is hidden by every run's waves together
@@ -333,7 +339,14 @@ extern "C" int awp_batch_create(awp_batch **out, awp_ctx *const *runs, int nruns
             rows += row_segments(runs[r]->g);
             nz = std::max(nz, runs[r]->g.nz);
         }
-        b->kc_split = split_kc(rows, nz);
+        if (b->l.staged) {
+            long long cols = 0;
+            for (int r = 0; r < nruns; ++r) cols += staged_cols(runs[r]->g);
+            const int n = staged_nchunk(cols, nz);
+            b->kc_split = (nz + n - 1) / n;
+        } else {
+            b->kc_split = split_kc(rows, nz);
+        }
     }
     b->d_jobs = nullptr;
     b->d_sjobs = nullptr;
@@ -473,13 +486,21 @@ extern "C" int awp_batch_tune(awp_batch *b, int reps)
         int ty, pf, nchunk;   // nchunk: z chunks per run (fused), chunk length in levels (two-stage)
         int xw;      // two-stage: waves per tile row
         int sform;   // two-stage stress kernel: 0 = 64-bit offsets, 1 = 32-bit offsets, 2 blocks per
-                     // CU; 2 = 32-bit offsets (0 and 2: blocks as registers allow)
+                     // CU; 2 = 32-bit offsets (0 and 2: blocks as registers allow); 3 = both kernels staged
         bool patch;  // two-stage: the runs' tile patches (else rows of tiles)
     };
     std::vector<Cand> cands;
     // two-stage, one block per tile, chunk lengths about the default's
     for (int kc : {b->kc_split * 2 / 3, b->kc_split, b->kc_split * 3 / 2})
         for (bool pt : {true, false}) cands.push_back({true, false, 4, 1, std::max(4, kc), 1, b->o32 ? 2 : 0, pt});
+    {
+        Launch sl = b->l;
+        sl.unroll = sl.tile_xw = 1;
+        sl.bpc_v = sl.bpc_s = 0;
+        if (staged_shape(sl))
+            for (int kc : {b->kc_split * 2 / 3, b->kc_split, b->kc_split * 3 / 2})
+                cands.push_back({true, false, STAGED_TY, 1, std::max(4, kc), 1, 3, true});
+    }
     for (bool ps : {true, false}) {
         // two-stage: tile rows x z chunk length (levels) x stress kernel form
         // x tile order
@@ -509,6 +530,7 @@ extern "C" int awp_batch_tune(awp_batch *b, int reps)
     auto apply_form = [b, spw0, sph0](int sf, bool patch) {
         b->l.o32_s = sf != 0;
         b->l.bpc_s = sf == 1 ? 2 : 0;
+        b->l.staged = sf == 3;
         b->l.spw = patch ? spw0 : 0;
         b->l.sph = patch ? sph0 : 0;
         set_block_caps(b->l, b->device);

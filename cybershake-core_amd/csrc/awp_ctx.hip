@@ -130,9 +130,10 @@ static bool want_fused(const Geo &g, int storage)
 
 // Whether a run that holds both buffers starts on the fused step: always
 // under AWP_SCHEME=fused, else from 200M points on.  FP32, two-stage against
-// fused on the same buffers: 200x200x100 0.20 against 0.23 ms per step,
-// 517x389x149 1.24 against 1.29, 800x600x200 3.60 against 3.74, 1500x1000x300
-// 17.1 against 16.8.
+// fused on the same buffers: 200x200x100 0.17 against 0.23 ms per step,
+// 517x389x149 1.13 against 1.29, 800x600x200 3.43 against 3.74; 1500x1000x300,
+// both tuned, 15.2 / 16.2 against 15.4 / 16.8 where the buffers lie well /
+// badly.
 static bool start_fused(const Geo &g)
 {
     const char *scheme = getenv("AWP_SCHEME");
@@ -292,6 +293,8 @@ static Launch choose_launch(const Geo &g, bool fused, bool mixed, int device)
             l.unroll = 0;
         }
     }
+    l.staged = false;
+    if (!fused) choose_staged(l, mixed);
     const long long bxy = (long long)((g.nx + TX - 1) / TX) * ((g.ny + l.tile_y - 1) / l.tile_y);
     int nchunk;
     if (fused && l.tile_y == 11) {
@@ -311,7 +314,7 @@ static Launch choose_launch(const Geo &g, bool fused, bool mixed, int device)
         nchunk = 2 * std::max(1, (g.nz + 75) / 150);
         nchunk = std::min(nchunk, std::max(1, g.nz / 16));
     } else {
-        nchunk = split_nchunk(g.nz, split_kc(row_segments(g), g.nz));
+        nchunk = l.staged ? staged_nchunk(staged_cols(g), g.nz) : split_nchunk(g.nz, split_kc(row_segments(g), g.nz));
     }
     const char *kc_env = getenv("AWP_KC");
     if (kc_env && atoi(kc_env) >= 3) nchunk = std::max(1, (g.nz + atoi(kc_env) - 1) / atoi(kc_env));
@@ -1067,28 +1070,39 @@ extern "C" int awp_tune(awp_ctx *ctx, int reps)
     HIPTRY(ctx, hipSetDevice(ctx->device));
     int rc = ensure_events(ctx, 2);
     if (rc) return rc;
-    // candidates: the two-stage step with its defaults, with shorter and
-    // longer z chunks and on taller tiles; with both buffers,
-    // the fused step on 64 x 11 tiles (FP32; z chunks of about 100, 75, 60
-    // levels x tile patches 4x4, 2x2, 8x2, and larger patches) and 64 x 8
-    // tiles, or on 64 x 7 tiles (mixed).  The fastest is kept.
+    // candidates: the two-stage step with its defaults and staged with shorter
+    // and longer z chunks (where staged is not its default: also without LDS,
+    // on other tiles and chunks); with both buffers, the fused step on 64 x 11
+    // tiles (FP32; z chunks of about 100 and 75 levels x tile patches 4x4,
+    // 2x2, 8x2, and larger patches) and 64 x 8 tiles, or on 64 x 7 tiles
+    // (mixed).  The fastest is kept.
     struct Cand {
         bool fused;
         int ty, kc, pw, ph;
+        bool staged = false;
     };
     std::vector<Cand> cands;
     cands.push_back({false, 0, 0, 0, 0});
     {
+        const Launch d = choose_launch(ctx->g, false, ctx->mixed(), ctx->device);
+        if (staged_shape(d)) {
+            const int n = staged_nchunk(staged_cols(ctx->g), ctx->g.nz), kc = (ctx->g.nz + n - 1) / n;
+            for (int q : {d.staged ? 0 : kc, std::max(4, kc * 2 / 3), kc * 3 / 2})
+                if (q) cands.push_back({false, STAGED_TY, q, 0, 0, true});
+        }
+        // the form without LDS where the staged one is not the default
         const int kc = split_kc(row_segments(ctx->g), ctx->g.nz);
-        cands.push_back({false, 4, std::max(4, kc * 2 / 3), 0, 0});
-        cands.push_back({false, 4, kc * 3 / 2, 0, 0});
-        cands.push_back({false, kc > 8 ? 2 : 4, kc, 0, 0});
-        cands.push_back({false, 8, 25, 0, 0});
+        if (!d.staged) {
+            cands.push_back({false, 4, std::max(4, kc * 2 / 3), 0, 0});
+            cands.push_back({false, 4, kc * 3 / 2, 0, 0});
+            cands.push_back({false, kc > 8 ? 2 : 4, kc, 0, 0});
+            cands.push_back({false, 8, 25, 0, 0});
+        }
     }
     if (ctx->two_bufs) {
         if (!ctx->mixed()) {
             const int pat[3][2] = {{4, 4}, {2, 2}, {8, 2}};
-            for (int kc : {100, 75, 60})
+            for (int kc : {100, 75})
                 for (const auto &pp : pat) cands.push_back({true, 11, kc, pp[0], pp[1]});
             // larger patches: more of an XCD's 32 resident tiles are
             // neighbours that share their halo lines
@@ -1114,8 +1128,10 @@ extern "C" int awp_tune(awp_ctx *ctx, int reps)
         ctx->fused = cd.fused;
         Launch l = choose_launch(ctx->g, cd.fused, ctx->mixed(), ctx->device);
         if (!cd.fused && cd.ty) {
+            l.staged = false;
             l.tile_y = cd.ty;
             l.tile_xw = 1;
+            if (cd.staged) set_staged(l);
             set_chunks(l, ctx->g, split_nchunk(ctx->g.nz, cd.kc), false);
         }
         if (cd.fused) {
@@ -1130,8 +1146,10 @@ extern "C" int awp_tune(awp_ctx *ctx, int reps)
     };
     // one warm-up step, then `reps` timed ones (ms in *ms)
     auto time_steps = [ctx, reps](float *ms) -> int { return time_trial(ctx, reps, ms); };
-    // the fastest of the candidates
+    // the fastest of the candidates; a run that starts fused stays so unless
+    // the two-stage step is faster by more than a twentieth
     size_t pick = 0;
+    const float lead = ctx->fused ? 1.05f : 1.0f;
     // AWP_TUNE_LOG=1: every timing on stderr
     const char *tl = getenv("AWP_TUNE_LOG");
     const bool log = tl && atoi(tl) == 1;
@@ -1146,9 +1164,9 @@ extern "C" int awp_tune(awp_ctx *ctx, int reps)
             if (r) return r;
             if (log)
                 fprintf(stderr, "awp_tune: %s ty %d kc %d patch %dx%d: %.3f ms per step\n",
-                        cands[n].fused ? "fused" : "two-stage", cands[n].ty, cands[n].kc, cands[n].pw, cands[n].ph,
+                        cands[n].fused ? "fused" : cands[n].staged ? "staged" : "two-stage", cands[n].ty, cands[n].kc, cands[n].pw, cands[n].ph,
                         ms / reps);
-            first.push_back({ms, n});
+            first.push_back({cands[n].fused ? ms : ms * lead, n});
         }
         std::sort(first.begin(), first.end());
         float best = 1e30f;
@@ -1162,10 +1180,11 @@ extern "C" int awp_tune(awp_ctx *ctx, int reps)
             if (r) return r;
             if (log)
                 fprintf(stderr, "awp_tune again: %s ty %d kc %d patch %dx%d: %.3f ms per step\n",
-                        cands[n].fused ? "fused" : "two-stage", cands[n].ty, cands[n].kc, cands[n].pw, cands[n].ph,
+                        cands[n].fused ? "fused" : cands[n].staged ? "staged" : "two-stage", cands[n].ty, cands[n].kc, cands[n].pw, cands[n].ph,
                         (ms + ms2) / (2 * reps));
-            if (ms + ms2 < best) {
-                best = ms + ms2;
+            const float both = (ms + ms2) * (cands[n].fused ? 1.0f : lead);
+            if (both < best) {
+                best = both;
                 pick = n;
             }
         }

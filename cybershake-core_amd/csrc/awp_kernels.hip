@@ -19,6 +19,8 @@
 #include "awp_kernels.hpp"
 
 #include <algorithm>
+#include <cstdlib>
+#include <cstring>
 
 namespace awp {
 
@@ -895,6 +897,33 @@ k_stress_batch(const SJob *__restrict__ jobs, const int njobs, const int total, 
     if (claim && threadIdx.x == 0 && threadIdx.y == 0 && threadIdx.z == 0) claim_done(claim, (int)gridDim.x);
 }
 
+}  // namespace awp
+#include "awp_staged.hpp"
+namespace awp {
+
+// the staged stages (awp_staged.hpp), one tile per block
+template <class P>
+__global__ void __launch_bounds__(TX * STAGED_TY)
+k_velocity_staged(const SJob *__restrict__ jobs, const int njobs, const int total, const int per, const Hook hook)
+{
+    const int tile = stage_tile(nullptr, per, total, 0, 0, nullptr);
+    if (tile < 0) return;
+    int bx, by, bz;
+    const SJob &J = split_tile(jobs, njobs, tile, bx, by, bz);
+    velocity_tile_s<P>(J.g, J.s, J.c, J.kc, bx, by, bz, hook);
+}
+template <class P>
+__global__ void __launch_bounds__(TX * STAGED_TY)
+k_stress_staged(const SJob *__restrict__ jobs, const int njobs, const int total, const int per, const int rot,
+                const Hook hook)
+{
+    const int tile = stage_tile(nullptr, per, total, rot, 0, nullptr);
+    if (tile < 0) return;
+    int bx, by, bz;
+    const SJob &J = split_tile(jobs, njobs, tile, bx, by, bz);
+    stress_tile_s<P>(J.g, J.s, J.c, J.kc, bx, by, bz, hook);
+}
+
 // ---------------------------------------------------------------------------
 // point source, addsrc (source.f:812-913).  One thread walks the sources in
 // file order so coincident sources accumulate in the reference's order.
@@ -1435,6 +1464,45 @@ hipError_t launch_sgt_gather(const State &s, int nkept, const long long *kpos, c
     return hipGetLastError();
 }
 
+bool staged_shape(const Launch &l)
+{
+    const char *e = getenv("AWP_STAGED");
+    return l.o32 && l.o32_s && l.unroll == 1 && l.tile_xw == 1 && !l.bpc_v && !l.bpc_s && !l.claim &&
+           !(e && !strcmp(e, "0"));
+}
+
+// 3 x 2 tile patches: 1500x1000x300 FP32 16.29 ms per step against 16.36 (3 x
+// 8), 16.38 (3 x 4) and 16.47 (rows); mixed the same within 1 %
+void set_staged(Launch &l)
+{
+    l.staged = true;
+    l.tile_y = STAGED_TY;
+    if (getenv("AWP_SPATCH")) return;
+    l.spw = 3;
+    l.sph = 2;
+}
+
+// The staged form unless the run fits the memory-side cache whole, or (mixed)
+// all of it but r1..r6: there a step is bound by the chain of a wave's
+// levels, which the barrier of each lengthens.  us per step without / with,
+// FP32: 48x40x32 27 / 32, 150x150x90 79 / 89, 180x160x90 (mode 2) 111 / 102,
+// 203x187x101 168 / 163, 240x220x80 171 / 152, 260x220x100 267 / 237,
+// 517x389x149 1219 / 1132, 800x600x200 3595 / 3430, 1500x1000x300 17194 /
+// 16292; mixed: 48x40x32 32 / 38, 150x150x90 78 / 97, 180x160x90 89 / 100,
+// 200x200x100 (mode 2) 156 / 150, 203x187x101 148 / 153, 240x220x80 145 / 143,
+// 260x220x100 (mode 3) 224 / 221, 250x250x110 240 / 214, 517x389x149 1023 /
+// 951, 800x600x200 2961 / 2821, 1500x1000x300 14157 / 13342.  AWP_STAGED=1
+// takes it wherever the shape admits it, 0 nowhere; a tile height
+// (AWP_TILE_Y) other than its own asks for the other form.
+void choose_staged(Launch &l, bool mixed)
+{
+    const char *e = getenv("AWP_STAGED"), *ty = getenv("AWP_TILE_Y");
+    l.staged = false;
+    if (!staged_shape(l) || (ty && atoi(ty) != STAGED_TY)) return;
+    const bool gains = mixed ? l.cached == 0 || l.cached == 3 : l.cached != 1;
+    if (gains || (e && !strcmp(e, "1"))) set_staged(l);
+}
+
 void set_block_caps(Launch &l, int device)
 {
     int cu = 0, blk = 0;
@@ -1572,12 +1640,50 @@ static hipError_t stress_stage(const Launch &l, bool os, const SJob *d_jobs, int
     return hipSuccess;
 }
 
+template <class P>
+static void staged_velocity(const SJob *d_jobs, int njobs, int total, int per, const Hook &hook, hipStream_t st)
+{
+    hipLaunchKernelGGL((k_velocity_staged<P>), dim3(8 * per), dim3(TX, STAGED_TY), 0, st, d_jobs, njobs, total, per,
+                       hook);
+}
+template <class P>
+static void stress_staged(const SJob *d_jobs, int njobs, int total, int per, int rot, const Hook &hook, hipStream_t st)
+{
+    hipLaunchKernelGGL((k_stress_staged<P>), dim3(8 * per), dim3(TX, STAGED_TY), 0, st, d_jobs, njobs, total, per, rot,
+                       hook);
+}
+// (the other way round beyond the cache modes, as str_batch_t)
+template <class P>
+static void staged_stress(const Launch &l, const SJob *d_jobs, int njobs, int total, int per, const Hook &hook,
+                          hipStream_t st)
+{
+    if (l.cached == 0)
+        stress_staged<P>(d_jobs, njobs, total, per, 8, hook, st);
+    else if (l.cached == 1)
+        stress_staged<Cached<P, 0>>(d_jobs, njobs, total, per, 0, hook, st);
+    else if (l.cached == 2)
+        stress_staged<Cached<P, 1>>(d_jobs, njobs, total, per, 0, hook, st);
+    else
+        stress_staged<Cached<P, 2>>(d_jobs, njobs, total, per, 0, hook, st);
+}
+
 hipError_t launch_split_velocity(bool mixed, const Launch &l, bool o32, const SJob *d_jobs, int njobs, int total,
                                  int grid_v, unsigned long long *claim, const Hook &hook, hipStream_t st)
 {
     if (njobs <= 0 || total <= 0) return hipSuccess;
     const int per = (total + 7) / 8;
     const bool ov = o32 && l.o32_v;
+    if (l.staged) {
+        if (mixed && l.cached)
+            staged_velocity<Cached<StoreMixed, 0>>(d_jobs, njobs, total, per, hook, st);
+        else if (mixed)
+            staged_velocity<StoreMixed>(d_jobs, njobs, total, per, hook, st);
+        else if (l.cached)
+            staged_velocity<Cached<StoreF32, 0>>(d_jobs, njobs, total, per, hook, st);
+        else
+            staged_velocity<StoreF32>(d_jobs, njobs, total, per, hook, st);
+        return hipGetLastError();
+    }
     if (l.cached && l.unroll != 2 && !tall(l)) {
         if (mixed) vel_batch_t<Cached<StoreMixed, 0>, 1, 512>(l, ov, d_jobs, njobs, total, per, grid_v, claim, hook, st);
         else vel_batch_t<Cached<StoreF32, 0>, 1, 512>(l, ov, d_jobs, njobs, total, per, grid_v, claim, hook, st);
@@ -1595,6 +1701,13 @@ hipError_t launch_split_stress(bool mixed, const Launch &l, bool o32, const SJob
     if (njobs <= 0 || total <= 0) return hipSuccess;
     const int per = (total + 7) / 8;
     const bool os = o32 && l.o32_s;
+    if (l.staged) {
+        if (mixed)
+            staged_stress<StoreMixed>(l, d_jobs, njobs, total, per, hook, st);
+        else
+            staged_stress<StoreF32>(l, d_jobs, njobs, total, per, hook, st);
+        return hipGetLastError();
+    }
     if (l.cached && os && l.unroll != 2 && !tall(l)) {
         if (mixed) cached_stress<StoreMixed>(l, d_jobs, njobs, total, per, grid_s, claim, hook, st);
         else cached_stress<StoreF32>(l, d_jobs, njobs, total, per, grid_s, claim, hook, st);

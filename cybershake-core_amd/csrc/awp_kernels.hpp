@@ -405,10 +405,19 @@ struct Cursor32 {
     {
         gsn<NT>(p, o >> (sizeof(T) == 2 ? 1 : 0), v);
     }
+    // the point dk levels up, streamed
+    template <bool NT, class T>
+    __device__ __forceinline__ T ldu(const G<T> *p, int dk) const
+    {
+        return gln<NT>(p, at(0, dk) >> (sizeof(T) == 2 ? 1 : 0));
+    }
     __device__ __forceinline__ void up() { o += sz; }
 };
 
-// z chunk length of the two-stage kernels for `rows` row segments of 64
+// rows of a staged two-stage tile (awp_staged.hpp)
+constexpr int STAGED_TY = 8;
+
+// z chunk length of the two-stage kernels without LDS for `rows` row segments of 64
 // points a level and nz levels.  A wave marches its chunk level by level, 2.9
 // us each on an idle GPU (load, compute, store), so a grid that cannot fill
 // the GPU's 4096 wave slots (4 per SIMD) is bound by that chain and takes
@@ -436,6 +445,40 @@ static inline int split_nchunk(int nz, int kc)
 {
     const int n = (nz + kc / 2) / kc;
     return n < 1 ? 1 : n;
+}
+
+// z chunks of the staged two-stage kernels: `cols` tiles of 64 x STAGED_TY
+// points a level (of every run of a step), nz levels.  512 blocks of the
+// stress kernel are on the GPU at once (two a CU, by its registers), so a
+// step takes `rounds` times a chunk's levels and about one for its start-up
+// loads: the chunks that make the least of it, at most 30 levels each
+// (longer ones drift apart and share less in the caches: 1500x1000x300 with
+// 25 / 75 / 150 levels 16.32 / 16.72 / 17.33 ms per step).  Beyond a few
+// rounds the blocks spread, and half a round more than the mean is lost
+// instead of a whole one.  us per step, FP32 / mixed: 200x200x100 with 5 / 6 /
+// 9 / 10 chunks 167 / 188 / 185 / 168 and 150 / 184 / 172 / 153; 300x300x120
+// with 6 / 8 / 10 / 12 439 / 412 / 422 / 414 and 381 / 346 / 362 / 356;
+// 517x389x149 with 6 / 8 / 11 / 13 1171 / 1132 / 1193 / 1165 and 984 / 951 /
+// 990 / 997.
+static inline int staged_nchunk(long long cols, int nz)
+{
+    int best = 1;
+    double least = 1e30;
+    for (int n = (nz + 29) / 30; n <= (nz + 3) / 4; ++n) {
+        const double x = (double)n * (double)cols / 512;
+        const double rounds = x > 8 ? x + 0.5 : (double)(long long)(x + 0.999999);
+        const double cost = rounds * ((nz + n - 1) / n + 1);
+        if (cost < least) {
+            least = cost;
+            best = n;
+        }
+    }
+    return best;
+}
+// tiles a level of a grid
+static inline long long staged_cols(const Geo &g)
+{
+    return (long long)((g.nx + 63) / 64) * ((g.ny + STAGED_TY - 1) / STAGED_TY);
 }
 
 // What of nvol points' step arrays the two-stage kernels keep in the 256 MB
@@ -503,6 +546,7 @@ struct Launch {
     bool o32;        // 32-bit byte offsets reach every array (offsets32() of the run's geometry)
     bool o32_s;      // two-stage stress kernel: its 32-bit byte-offset form (only where o32)
     int cached;      // two-stage kernels: cache_mode() of the run
+    bool staged;     // two-stage kernels: the staged form (awp_staged.hpp): 64 x STAGED_TY tiles, one per block, o32
     bool o32_v;      // two-stage velocity kernel: its 32-bit byte-offset form (only where o32)
     int bpc_v, bpc_s;   // two-stage kernels: most blocks per CU (0 = as registers allow)
     unsigned lds_v, lds_s;   // the dynamic LDS bytes per block that enforce them (set_block_caps)
@@ -519,6 +563,11 @@ static inline unsigned lds_cap(int bpc, int lds_cu, int lds_block)
     const int want = lds_cu / bpc - 512;
     return (want > 0 && want <= lds_block) ? (unsigned)want : 0u;
 }
+// whether a two-stage launch shape admits the staged form, and the shape of it
+bool staged_shape(const Launch &l);
+void set_staged(Launch &l);
+// set_staged where a default shape gains by it
+void choose_staged(Launch &l, bool mixed);
 // fills lds_v / lds_s of `l` from bpc_v / bpc_s for device `device`
 void set_block_caps(Launch &l, int device);
 
