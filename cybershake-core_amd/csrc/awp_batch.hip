@@ -314,7 +314,7 @@ extern "C" int awp_batch_create(awp_batch **out, awp_ctx *const *runs, int nruns
     } else {
         b->l.tile_y = (b->l.tile_y == 4 || b->l.tile_y == 7 || b->l.tile_y == 8 || b->l.tile_y == 11) ? b->l.tile_y
                                                                                                      : 8;
-        // 64 x 8: no prefetch; 64 x 11: none, with one or two levels per barrier
+        // 64 x 8: no prefetch; 64 x 11: none or variant 3
         if (b->l.tile_y == 8 || (b->l.tile_y == 11 && b->l.unroll != 3)) b->l.unroll = 0;
         b->l.tile_xw = 1;
     }
@@ -338,6 +338,14 @@ extern "C" int awp_batch_create(awp_batch **out, awp_ctx *const *runs, int nruns
         for (int r = 0; r < nruns; ++r) {
             rows += row_segments(runs[r]->g);
             nz = std::max(nz, runs[r]->g.nz);
+        }
+        if (!b->split && !b->mixed && b->l.tile_y == 11 && b->l.unroll == 3) {
+            long long cols = 0;
+            for (int r = 0; r < nruns; ++r) {
+                const FTiles t = fused_tiles(runs[r]->g, b->l);
+                cols += (long long)t.nbx * t.nby;
+            }
+            b->nchunk.assign(nruns, sweep_nchunk(cols, nz));
         }
         if (b->l.staged) {
             long long cols = 0;

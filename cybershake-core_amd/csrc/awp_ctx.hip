@@ -115,10 +115,9 @@ static void place_arrays(awp_ctx *ctx)
 // one-sweep fused step (a second wavefield buffer; every array addressed
 // with 32-bit byte offsets from a base rebased per z chunk, so chunks of at
 // most fused_kc_max levels).  Unset: fused for FP32 storage, two-stage for
-// mixed storage (1500x1000x300, one run's buffers: fused FP32 16.8-16.9 ms
-// per step on 64 x 11 tiles against 17.2-17.3 two-stage; fused mixed 23.7
-// against 14.7).  awp_tune
-// and awp_set_scheme switch a run that holds both buffers between the two.
+// mixed storage (1500x1000x300, one run's buffers: fused FP32 14.6 ms per step
+// on 64 x 11 tiles against 16.3 two-stage; fused mixed 21.5 against 13.3).
+// awp_tune and awp_set_scheme switch a run that holds both buffers between the two.
 static bool want_fused(const Geo &g, int storage)
 {
     if (fused_kc_max(g) < 16) return false;   // planes of more than ~40M points
@@ -129,15 +128,15 @@ static bool want_fused(const Geo &g, int storage)
 }
 
 // Whether a run that holds both buffers starts on the fused step: always
-// under AWP_SCHEME=fused, else from 200M points on.  FP32, two-stage against
-// fused on the same buffers: 200x200x100 0.17 against 0.23 ms per step,
-// 517x389x149 1.13 against 1.29, 800x600x200 3.43 against 3.74; 1500x1000x300,
-// both tuned, 15.2 / 16.2 against 15.4 / 16.8 where the buffers lie well /
-// badly.
+// under AWP_SCHEME=fused, else from 25M points on (below, a tile a CU leaves
+// too few rounds to even out).  FP32, two-stage against fused on the same
+// buffers, us per step: 200x200x100 165 against 196, 300x300x120 414 against
+// 428, 517x389x149 (30M) 1133 against 1101, 800x600x200 3430 against 3193,
+// 1500x1000x300 16290 against 14640.
 static bool start_fused(const Geo &g)
 {
     const char *scheme = getenv("AWP_SCHEME");
-    return (scheme && !strcmp(scheme, "fused")) || (long long)g.nx * g.ny * g.nz >= 200000000ll;
+    return (scheme && !strcmp(scheme, "fused")) || (long long)g.nx * g.ny * g.nz >= 25000000ll;
 }
 
 // z chunks of `nchunk` requested: the top chunk keeps >= 3 levels (the
@@ -187,30 +186,29 @@ static Launch choose_launch(const Geo &g, bool fused, bool mixed, int device)
     // the two-stage kernels, 4, 7, 8 or 11 for the fused one) and AWP_KC (z
     // levels per block)
     const char *ty = getenv("AWP_TILE_Y");
-    // fused defaults measured at 1500x1000x300: FP32 64x11 tiles (16-wave
-    // blocks fill a CU's wave slots: 16.2-16.3 ms per step against 17.7-18.1
-    // for 64x8), mixed 64x7 tiles, both without load prefetch (awp_tune and
-    // awp_batch_tune search the rest)
+    // fused defaults: FP32 64x11 tiles (awp_sweep.hpp; 16-wave blocks fill a
+    // CU's wave slots: 14.6 ms per step at 1500x1000x300 against 17.3 for the
+    // same tiles without it), mixed 64x7 tiles without load prefetch
     if (fused) l.tile_y = mixed ? 7 : 11;
     if (ty && (atoi(ty) == 1 || atoi(ty) == 2 || atoi(ty) == 4 || atoi(ty) == 7 || atoi(ty) == 8 || atoi(ty) == 11 ||
                atoi(ty) == 16))
         l.tile_y = atoi(ty);
     if (fused && l.tile_y != 4 && l.tile_y != 7 && l.tile_y != 11) l.tile_y = 8;
     if (!fused && (l.tile_y == 7 || l.tile_y == 11)) l.tile_y = 8;
-    // tile patches of the fused step (AWP_PATCH=<w>x<h> overrides): 4 x 4
-    // tiles of 64 x 8 points (1500x1000x300 FP32, 4 z chunks: 17.21 ms per
-    // step against 17.62 for 2 x 16 and 17.75 for 3 x 8)
-    l.pw = 4;
-    l.ph = 4;
+    // tile patches of the fused step (AWP_PATCH=<w>x<h> overrides): FP32 64 x
+    // 11 2 x 2 (1500x1000x300: 14.64 ms per step against 14.72 for 4 x 4, 14.88
+    // for 8 x 2, 15.06 for rows and 15.14 for 3 x 3), else 4 x 4 (64 x 8, 4 z
+    // chunks: 17.21 against 17.62 for 2 x 16 and 17.75 for 3 x 8)
+    l.pw = l.ph = fused && l.tile_y == 11 && !mixed ? 2 : 4;
     // tile claim (AWP_CLAIM=0 never, 1 when the launch has at least four
     // tiles per persistent block, 2 always; AWP_XROT=0..7 rotates the XCD
-    // ranges): persistent blocks that claim tiles per XCD.  The fused step's
-    // default (1500x1000x300: 16.81-16.92 ms per step against 17.11-17.20
-    // with one block per tile, same run); the two-stage kernels run one block
-    // per tile, whose dispatch costs less than a claim per short tile
-    // (400x300x150, 64 x 2 tiles of 17 levels: 0.749 ms per step against
-    // 0.923 claimed)
-    l.claim = fused ? 1 : 0;
+    // ranges): persistent blocks that claim tiles per XCD.  The default of
+    // the fused step without awp_sweep.hpp (1500x1000x300: 16.81-16.92 ms per
+    // step against 17.11-17.20 with one block per tile, same run); with it
+    // (14.70 against 14.85 claimed) and in the two-stage kernels (400x300x150,
+    // 64 x 2 tiles of 17 levels: 0.749 against 0.923 claimed) one block per
+    // tile, whose dispatch costs less than a claim
+    l.claim = fused && (mixed || l.tile_y != 11) ? 1 : 0;
     l.xrot = 0;
     const char *ce = getenv("AWP_CLAIM");
     if (ce && (!strcmp(ce, "0") || !strcmp(ce, "1") || !strcmp(ce, "2"))) l.claim = ce[0] - '0';
@@ -283,9 +281,8 @@ static Launch choose_launch(const Geo &g, bool fused, bool mixed, int device)
     if (fused) {
         // the fused step keeps its load prefetch depth (0, 1, 2) in `unroll`
         const char *pf = getenv("AWP_PF");
-        // (3: no prefetch, two levels per barrier, on 64 x 11 tiles only --
-        // their default: 1500x1000x300 16.17-16.27 ms per step against
-        // 16.48-16.58 with one level per barrier on the same buffers)
+        // (3, the default of 64 x 11 tiles and theirs only: FP32
+        // awp_sweep.hpp, mixed two levels per barrier without prefetch)
         l.unroll = (pf && atoi(pf) >= 0 && atoi(pf) <= 3) ? atoi(pf) : (l.tile_y == 11 ? 3 : 0);
         if (l.tile_y == 11) {
             if (l.unroll != 0 && l.unroll != 3) l.unroll = 3;
@@ -297,11 +294,13 @@ static Launch choose_launch(const Geo &g, bool fused, bool mixed, int device)
     if (!fused) choose_staged(l, mixed);
     const long long bxy = (long long)((g.nx + TX - 1) / TX) * ((g.ny + l.tile_y - 1) / l.tile_y);
     int nchunk;
-    if (fused && l.tile_y == 11) {
+    if (fused && l.tile_y == 11 && !mixed && l.unroll == 3) {
+        nchunk = sweep_nchunk(bxy, g.nz);
+    } else if (fused && l.tile_y == 11) {
         // chunks of about 100 levels: at 1500x1000x300 with 4 x 4 patches,
-        // 3 chunks ran 16.21-16.23 ms per step on two boxes; 4 chunks
-        // 16.34 on one and 17.71 on the other, 2 chunks 17.92 (each chunk
-        // recomputes 4 velocity levels)
+        // 3 chunks ran 16.21-16.23 ms per step, 4 chunks 16.34 or 17.71 by
+        // where the buffers lay, 2 chunks 17.92 (each chunk recomputes 4
+        // velocity levels)
         // Grids of few tile columns take more chunks, four tiles per CU
         // (517x389x149, 324 columns: one chunk 1.66 ms per step, two 1.37,
         // three 1.29, six 1.29)
@@ -1073,8 +1072,7 @@ extern "C" int awp_tune(awp_ctx *ctx, int reps)
     // candidates: the two-stage step with its defaults and staged with shorter
     // and longer z chunks (where staged is not its default: also without LDS,
     // on other tiles and chunks); with both buffers, the fused step on 64 x 11
-    // tiles (FP32; z chunks of about 100 and 75 levels x tile patches 4x4,
-    // 2x2, 8x2, and larger patches) and 64 x 8 tiles, or on 64 x 7 tiles
+    // tiles (FP32; other tile patches and z chunks) or on 64 x 7 tiles
     // (mixed).  The fastest is kept.
     struct Cand {
         bool fused;
@@ -1101,24 +1099,11 @@ extern "C" int awp_tune(awp_ctx *ctx, int reps)
     }
     if (ctx->two_bufs) {
         if (!ctx->mixed()) {
-            const int pat[3][2] = {{4, 4}, {2, 2}, {8, 2}};
-            for (int kc : {100, 75})
-                for (const auto &pp : pat) cands.push_back({true, 11, kc, pp[0], pp[1]});
-            // larger patches: more of an XCD's 32 resident tiles are
-            // neighbours that share their halo lines
-            const int big[3][2] = {{4, 8}, {8, 4}, {6, 5}};
-            for (const auto &pp : big) cands.push_back({true, 11, 100, pp[0], pp[1]});
-            cands.push_back({true, 11, 75, 3, 3});
-            // two chunks: less velocity recomputed at chunk edges
-            cands.push_back({true, 11, 150, 4, 4});
-            cands.push_back({true, 11, 150, 2, 2});
-            cands.push_back({true, 8, 75, 4, 4});
-            // small grids: more z chunks, or 64 x 4 tiles, for more tiles
-            const long long fxy = (long long)((ctx->g.nx + TX - 1) / TX) * ((ctx->g.ny + 10) / 11);
-            if (fxy * std::max(1, ctx->g.nz / 100) < 4096) {
-                for (int kc : {25, 16}) cands.push_back({true, 11, kc, 2, 2});
-                cands.push_back({true, 4, 16, 4, 4});
-            }
+            const int kc = choose_launch(ctx->g, true, false, ctx->device).kc;
+            const int pat[4][2] = {{2, 2}, {4, 4}, {2, 4}, {8, 2}};
+            for (const auto &pp : pat) cands.push_back({true, 11, kc, pp[0], pp[1]});
+            for (int k : {100, 75, 150, 25})
+                if (k < ctx->g.nz) cands.push_back({true, 11, k, 2, 2});
         } else {
             cands.push_back({true, 7, 75, 4, 4});
         }
@@ -1136,7 +1121,7 @@ extern "C" int awp_tune(awp_ctx *ctx, int reps)
         }
         if (cd.fused) {
             l.tile_y = cd.ty;
-            l.unroll = cd.ty == 11 ? 3 : 0;   // 64 x 11: two levels per barrier
+            l.unroll = cd.ty == 11 ? 3 : 0;
             l.pw = cd.pw;
             l.ph = cd.ph;
             set_chunks(l, ctx->g, std::min((ctx->g.nz + cd.kc / 2) / cd.kc, std::max(1, ctx->g.nz / 16)), true);
@@ -1146,10 +1131,8 @@ extern "C" int awp_tune(awp_ctx *ctx, int reps)
     };
     // one warm-up step, then `reps` timed ones (ms in *ms)
     auto time_steps = [ctx, reps](float *ms) -> int { return time_trial(ctx, reps, ms); };
-    // the fastest of the candidates; a run that starts fused stays so unless
-    // the two-stage step is faster by more than a twentieth
+    // the fastest of the candidates
     size_t pick = 0;
-    const float lead = ctx->fused ? 1.05f : 1.0f;
     // AWP_TUNE_LOG=1: every timing on stderr
     const char *tl = getenv("AWP_TUNE_LOG");
     const bool log = tl && atoi(tl) == 1;
@@ -1166,7 +1149,7 @@ extern "C" int awp_tune(awp_ctx *ctx, int reps)
                 fprintf(stderr, "awp_tune: %s ty %d kc %d patch %dx%d: %.3f ms per step\n",
                         cands[n].fused ? "fused" : cands[n].staged ? "staged" : "two-stage", cands[n].ty, cands[n].kc, cands[n].pw, cands[n].ph,
                         ms / reps);
-            first.push_back({cands[n].fused ? ms : ms * lead, n});
+            first.push_back({ms, n});
         }
         std::sort(first.begin(), first.end());
         float best = 1e30f;
@@ -1182,9 +1165,8 @@ extern "C" int awp_tune(awp_ctx *ctx, int reps)
                 fprintf(stderr, "awp_tune again: %s ty %d kc %d patch %dx%d: %.3f ms per step\n",
                         cands[n].fused ? "fused" : cands[n].staged ? "staged" : "two-stage", cands[n].ty, cands[n].kc, cands[n].pw, cands[n].ph,
                         (ms + ms2) / (2 * reps));
-            const float both = (ms + ms2) * (cands[n].fused ? 1.0f : lead);
-            if (both < best) {
-                best = both;
+            if (ms + ms2 < best) {
+                best = ms + ms2;
                 pick = n;
             }
         }

@@ -10,6 +10,8 @@
 // every array is read once and written once per step:
 //   FP32 storage: 140 B per point-update (176 B for the two-stage step)
 //   mixed storage: 116 B (FP16 r1..r6 under per-row exponents, FP16 qp/qs).
+// FP32 runs of at least 25M points take it by default, on 64 x 11 tiles
+// through awp_sweep.hpp; what follows here are the other tiles and storage.
 //
 // Stresses at the tile's edge need new velocities of the neighbouring tiles
 // (two columns / rows on each side).  The block recomputes them: its waves
@@ -29,7 +31,7 @@
 // two-stage kernels, which follow the reference CPU solver (operator.f:92-306,
 // viscoop.f:49-191, cerjan.f:249-328), so results are bit-identical to them.
 
-#include "awp_kernels.hpp"
+#include "awp_sweep.hpp"
 
 #include <algorithm>
 
@@ -87,8 +89,9 @@ struct StrIn {
 // what it needs; 1 = the stress stage's loads are issued before the velocity
 // stage's arithmetic; 2 = as 1, and the next level's velocity loads are
 // issued before the stress arithmetic.
-// PFC = 3: no prefetch, and the velocities of two levels per barrier (then
-// the stresses of two levels), which halves the block's barriers.
+// PFC = 3: mixed, no prefetch, and the velocities of two levels per barrier
+// (then the stresses of two levels), which halves the block's barriers; FP32
+// on 64 x 11 tiles, sweep_tile.
 // One column tile (bx, by, z chunk bz) of one run: the whole block calls it.
 // The volume arrays of s advanced by `e` elements (the sponge profiles and
 // the exponent slots keep their own indexing).
@@ -126,6 +129,12 @@ __device__ __forceinline__ GState rebased(const State &s0, const long long e)
     return s;
 }
 
+// the FP32 64 x 11 tile of variant 3 runs sweep_tile
+template <class P, int TY, int PFC>
+constexpr bool swept = !P::mixed && TY == Sweep::TY && PFC == 3;
+template <class P, int TY, int PFC>
+constexpr int lds_floats = swept<P, TY, PFC> ? Sweep::FLOATS : FShape<TY, PFC>::NSLOT * FShape<TY, PFC>::SLOT;
+
 template <class P, int TY, int PFC>
 __device__ __forceinline__ void step_tile(const Geo &g, const State &a0, const State &b0, const Coef &c,
                                           const int kc, const int bx, const int by, const int bz, float *lds)
@@ -134,6 +143,10 @@ __device__ __forceinline__ void step_tile(const Geo &g, const State &a0, const S
     const int lz = max(bz * kc + 1 - 4, -1);
     const long long rb = (long long)lz * g.sz;
     const GState a = rebased<P>(a0, rb), b = rebased<P>(b0, rb);
+    if constexpr (swept<P, TY, PFC>) {
+        sweep_tile(g, a, b, c, kc, bx, by, bz, rb, lds);
+        return;
+    } else {
     using Sh = FShape<TY, PFC>;
     constexpr int PF = PFC == 3 ? 0 : PFC;   // prefetch depth
     constexpr int LV = PFC == 3 ? 2 : 1;     // levels per barrier
@@ -634,14 +647,14 @@ __device__ __forceinline__ void step_tile(const Geo &g, const State &a0, const S
             if (two) str_level(m + 1, old1, sin1);
         }
     }
+    }
 }
 
 template <class P, int TY, int PF>
 __global__ void __launch_bounds__(64 * (TY + 5))
 k_step(const Geo g, const State a, const State b, const Coef c, const int kc, const FTiles tl)
 {
-    using Sh = FShape<TY, PF>;
-    __shared__ float lds[Sh::NSLOT * Sh::SLOT];
+    __shared__ __attribute__((aligned(16))) float lds[lds_floats<P, TY, PF>];
     int bx, by, bz;
     if (!ftile_of(tl, bx, by, bz)) return;   // uniform over the block
     step_tile<P, TY, PF>(g, a, b, c, kc, bx, by, bz, lds);
@@ -659,8 +672,7 @@ __global__ void __launch_bounds__(64 * (TY + 5))
 k_step_batch(const FJob *__restrict__ jobs, const int njobs, const int total, const int per, const int par,
              unsigned long long *claim, const int rot)
 {
-    using Sh = FShape<TY, PF>;
-    __shared__ float lds[Sh::NSLOT * Sh::SLOT];
+    __shared__ __attribute__((aligned(16))) float lds[lds_floats<P, TY, PF>];
     __shared__ int next;
     const bool lead = threadIdx.x == 0 && threadIdx.y == 0;
     for (;;) {

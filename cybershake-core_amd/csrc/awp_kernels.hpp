@@ -26,6 +26,7 @@
 // shifts the wave speeds coherently and took the SGT error past 1e-3).
 // Arithmetic is FP32 in both modes.
 #pragma once
+#include <algorithm>
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -510,6 +511,27 @@ static inline int fused_kc_max(const Geo &g)
 {
     const long long lv = (long long)(((1ull << 32) - 1) / (unsigned long long)(g.sz * 4));
     return (int)(lv - 10 > 1 << 20 ? 1 << 20 : lv - 10);
+}
+
+// z chunks of the FP32 fused step on 64 x 11 tiles (`cols` tiles a level): 256
+// blocks are on the GPU at once, one a CU, and a chunk recomputes four levels
+// of velocities, so n chunks take ceil(n cols / 256) (nz / n + 4) levels' time.
+// us per step at n chunks: 517x389x149 1 / 2 / 3 / 4 / 5 / 6 1403 / 1168 / 1101
+// / 1165 / 1137 / 1132, 800x600x200 1 / 2 / 3 / 4 3193 / 3248 / 3274 / 3298,
+// 300x300x120 3 / 4 / 5 / 6 / 7 / 8 442 / 486 / 428 / 460 / 436 / 450,
+// 1500x1000x300 2 / 3 / 4 / 5 14980 / 14637 / 14701 / 14697.
+static inline int sweep_nchunk(long long cols, int nz)
+{
+    int best = 1;
+    long long least = 1ll << 60;
+    for (int n = 1; n <= std::max(1, nz / 16); ++n) {
+        const long long cost = (n * cols + 255) / 256 * ((nz + n - 1) / n + 4);
+        if (cost < least) {
+            least = cost;
+            best = n;
+        }
+    }
+    return best;
 }
 
 // whether 32-bit byte offsets reach every element of a run's arrays (the
