@@ -9,8 +9,8 @@ Qs = 50 Vs[km/s], Qp = 2 Qs; X point force with a Gaussian source time
 function; 1.5M SGT points sampled every 10 steps.  Synthetic inputs are built
 on the device; the timed region is K full time steps with every input
 already resident in HBM.  A step is the two-stage one (velocity kernel,
-free-surface images, stress kernel with sponge and memory variables, source,
-SGT gather) or the one-sweep fused kernel in place of the first three: by
+stress kernel with free-surface images, sponge and memory variables, source,
+SGT gather) or the one-sweep fused kernel in place of the first two: by
 default (--scheme auto) the run takes the library's default scheme for its
 storage mode and awp_tune keeps the fastest scheme and launch shape before
 the warm-up; --scheme split / fused fixes the scheme at its default launch.
@@ -147,12 +147,12 @@ def bench_single(a, storage):
     ms_step = el / a.steps * 1e3
     kern_ms = ts / a.steps                   # fused kernel, or the stress kernel of the two-stage step
     if fused:
-        kname = ("k_step_batch (fused velocity + stress + sponge + free surface sweep over the run's one-entry "
-                 "job table; persistent blocks claiming tiles per XCD; k_step under AWP_CLAIM=0)")
+        kname = ("k_step (fused velocity + stress + sponge + free surface sweep, one block per tile; k_step_batch "
+                 "over the run's one-entry job table where AWP_CLAIM asks for claimed tiles)")
         bytes_pt = BYTES_UPDATE[storage]
         tname = "step_%s%s_traffic.txt" % (a.config, "" if storage == "fp32" else "_" + storage)
     else:
-        kname = "k_stress_batch (stress + memory variables + sponge + free surface; the run's one-entry job table)"
+        kname = "k_stress_staged (stress + memory variables + sponge + free surface; the run's one-entry job table)"
         bytes_pt = BYTES_STR[storage]
         tname = "stress_%s%s_traffic.txt" % (a.config, "" if storage == "fp32" else "_" + storage)
     ach = bytes_pt * npts_grid / (kern_ms * 1e-3) / 1e9
@@ -255,8 +255,8 @@ def bench_batched(a, storage, config=None, steps=None, warmup=None):
     roof = {"bound": "hbm",
             "kernel": ("whole batched step: k_step_batch (fused sweep over every run of a wave) + sources/SGT"
                        if fused else
-                       "whole batched step: k_velocity_batch + k_fs_velocity_batch + k_stress_batch (every run "
-                       "of a wave) + sources/SGT"),
+                       "whole batched step: k_velocity_staged + k_stress_staged (every run of a wave) + "
+                       "sources/SGT"),
             "achieved": round(ach, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(ach / HBM_PEAK_GBS, 4),
             "traffic": traffic_of(tname), "algorithmic_bytes_per_point": BYTES_UPDATE[storage],
             "algorithmic_bytes_per_step": int(BYTES_UPDATE[storage] * pts_step),

@@ -1,10 +1,9 @@
 // awp_batch.hip -- several SGT runs (components, sites) advanced together on
-// one GPU.  Each stage of a time step is one persistent launch over the
-// tiles of every run (a grid walking the concatenated tile list; the fused
-// kernel's blocks claim its tiles per XCD, claim_tile): in the
-// two-stage scheme the velocity kernel, the free-surface images and the
-// stress kernel, in the fused scheme the one-sweep kernel; then one launch
-// for every run's source and SGT sample.  Two steps (both buffer parities of
+// one GPU.  Each stage of a time step is one launch over the tiles of every
+// run: in the two-stage scheme the velocity and the stress kernel, one block
+// per tile of the concatenated list; in the fused scheme the one-sweep
+// kernel, whose persistent blocks claim the tiles per XCD (claim_tile); then
+// one launch for every run's source and SGT sample.  Two steps (both buffer parities of
 // the fused scheme) are captured in a HIP graph once and replayed.  The runs
 // keep their own contexts (buffers, counters, outputs): the batch only
 // drives them, so awp_get_sgt / awp_write_sgt_file work on each run
