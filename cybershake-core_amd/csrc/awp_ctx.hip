@@ -1261,39 +1261,80 @@ extern "C" int awp_device_bytes(const awp_ctx *ctx, size_t *bytes)
 // ---------------------------------------------------------------------------
 namespace {
 
-// Moves `bytes` of device memory through the run's pinned staging buffer in
-// order, in pieces of whole units (the last may be shorter): make(half, off,
-// n, &src) enqueues on the run's stream what produces bytes [off, off + n) and
-// says where they are, use(host, off, n) takes them on the host while the next
-// piece is on its way.  (A pageable copy runs at 10-17 GB/s through the
-// runtime's own staging, a pinned one at 57.)
+// The host memory one transfer of SGT output goes through: the run's pinned
+// buffer (two halves), or, where pinned memory is refused, pageable memory of
+// the transfer's own (one half).
 constexpr size_t PIN_HALF = (size_t)16 << 20;
 
-int drain_room(awp_ctx *ctx, size_t unit)
-{
-    const size_t half = std::max(PIN_HALF, unit);
-    for (int k = 0; k < 2; ++k)
-        if (!ctx->pin_ev[k]) HIPTRY(ctx, hipEventCreateWithFlags(&ctx->pin_ev[k], hipEventDisableTiming));
-    if (ctx->pin_half >= half) return AWP_OK;
-    if (ctx->pin) hipHostFree(ctx->pin);
-    ctx->pin = nullptr;
-    ctx->pin_half = 0;
-    const hipError_t e = hipHostMalloc((void **)&ctx->pin, 2 * half, hipHostMallocDefault);
-    if (e != hipSuccess) {
-        ctx->pin = nullptr;
-        return fail(ctx, AWP_ENOMEM, "hipHostMalloc(%zu): %s", 2 * half, hipGetErrorString(e));
+struct Stage {
+    char *host = nullptr;
+    size_t half = 0;
+    bool pinned = false;
+    Stage() = default;
+    Stage(const Stage &) = delete;
+    Stage &operator=(const Stage &) = delete;
+    ~Stage()
+    {
+        if (!pinned) free(host);
     }
-    ctx->pin_half = half;
-    return AWP_OK;
+};
+
+// the pinned buffer, if there is one whose halves hold a unit
+void pin_room(awp_ctx *ctx, size_t unit, Stage &s)
+{
+    if (!ctx->pin) {
+        const size_t half = std::max(PIN_HALF, unit);
+        char *p = nullptr;
+        bool ok = true;
+        for (hipEvent_t &ev : ctx->pin_ev)
+            if (!ev) ok = ok && hipEventCreateWithFlags(&ev, hipEventDisableTiming) == hipSuccess;
+        ok = ok && hipHostMalloc((void **)&p, 2 * half, hipHostMallocDefault) == hipSuccess;
+        if (!ok) {
+            (void)hipGetLastError();   // not the next call's error
+            return;
+        }
+        ctx->pin = p;
+        ctx->pin_half = half;
+    }
+    if (ctx->pin_half < unit) return;
+    s.host = ctx->pin;
+    s.half = ctx->pin_half;
+    s.pinned = true;
 }
 
-template <class MAKE, class USE>
-int drain(awp_ctx *ctx, size_t bytes, size_t unit, MAKE make, USE use)
+// staging of a transfer of `bytes` in whole units
+int stage_room(awp_ctx *ctx, size_t bytes, size_t unit, Stage &s)
 {
-    if (!bytes) return AWP_OK;
-    const int room = drain_room(ctx, unit);
-    if (room) return room;
-    const size_t half = ctx->pin_half, step = half / unit * unit;
+    pin_room(ctx, unit, s);
+    if (s.pinned) return AWP_OK;
+    s.half = std::max(std::min(PIN_HALF, bytes), unit);
+    s.host = (char *)malloc(s.half);
+    return s.host ? AWP_OK : fail(ctx, AWP_ENOMEM, "malloc(%zu) for the SGT output", s.half);
+}
+
+// Moves `bytes` of device memory through the staging s in order, in pieces of
+// whole units (the last may be shorter): make(half, off, n, &src) enqueues on
+// the run's stream what produces bytes [off, off + n) and says where they are,
+// use(host, off, n) takes them on the host, with pinned staging while the next
+// piece is on its way.  (A pageable copy runs at 10-17 GB/s through the
+// runtime's own staging, a pinned one at 57.)
+template <class MAKE, class USE>
+int drain(awp_ctx *ctx, const Stage &s, size_t bytes, size_t unit, MAKE make, USE use)
+{
+    const size_t half = s.half, step = half / unit * unit;
+    if (!s.pinned) {
+        for (size_t off = 0; off < bytes; off += step) {
+            const size_t n = std::min(step, bytes - off);
+            const void *src = nullptr;
+            int rc = make(0, off, n, &src);
+            if (rc) return rc;
+            HIPTRY(ctx, hipStreamSynchronize(ctx->stream));
+            HIPTRY(ctx, hipMemcpy(s.host, src, n, hipMemcpyDeviceToHost));
+            rc = use(s.host, off, n);
+            if (rc) return rc;
+        }
+        return AWP_OK;
+    }
     size_t sent = 0, done = 0;
     for (int k = 0; done < bytes; k ^= 1) {
         // keep one piece on its way beside the one in use
@@ -1302,14 +1343,17 @@ int drain(awp_ctx *ctx, size_t bytes, size_t unit, MAKE make, USE use)
             const size_t n = std::min(step, bytes - sent);
             const void *src = nullptr;
             int rc = make(h, sent, n, &src);
-            if (rc) return rc;
-            HIPTRY(ctx, hipMemcpyAsync(ctx->pin + h * half, src, n, hipMemcpyDeviceToHost, ctx->stream));
+            if (rc) {
+                hipStreamSynchronize(ctx->stream);   // as below
+                return rc;
+            }
+            HIPTRY(ctx, hipMemcpyAsync(s.host + h * half, src, n, hipMemcpyDeviceToHost, ctx->stream));
             HIPTRY(ctx, hipEventRecord(ctx->pin_ev[h], ctx->stream));
             sent += n;
         }
         const size_t n = std::min(step, bytes - done);
         HIPTRY(ctx, hipEventSynchronize(ctx->pin_ev[k]));
-        int rc = use(ctx->pin + k * half, done, n);
+        int rc = use(s.host + k * half, done, n);
         if (rc) {
             hipStreamSynchronize(ctx->stream);   // the piece on its way still lands in the buffer
             return rc;
@@ -1356,12 +1400,14 @@ extern "C" int awp_get_sgt(awp_ctx *ctx, float *host, size_t count)
     const size_t n = (size_t)ctx->npts * 6 * ctx->nsamp_max;
     if (count < n) return fail(ctx, AWP_EINVAL, "buffer holds %zu floats, need %zu", count, n);
     HIPTRY(ctx, hipSetDevice(ctx->device));
-    if (n * sizeof(float) < ((size_t)8 << 20)) {
+    Stage stage;
+    if (n * sizeof(float) >= ((size_t)8 << 20)) pin_room(ctx, 64, stage);
+    if (!stage.pinned) {
         HIPTRY(ctx, hipStreamSynchronize(ctx->stream));
         if (n) HIPTRY(ctx, hipMemcpy(host, ctx->d_sgt, n * sizeof(float), hipMemcpyDeviceToHost));
         return AWP_OK;
     }
-    return drain(ctx, n * sizeof(float), 64,
+    return drain(ctx, stage, n * sizeof(float), 64,
                  [ctx](int, size_t off, size_t, const void **src) {
                      *src = (const char *)ctx->d_sgt + off;
                      return AWP_OK;
@@ -1428,10 +1474,13 @@ extern "C" int awp_write_sgt_file(awp_ctx *ctx, const char *path)
         free(img);
     };
     int rc = AWP_OK;
-    if (e != hipSuccess) {
+    Stage stage;
+    if (e != hipSuccess)
         rc = fail(ctx, AWP_EHIP, "hipSetDevice: %s", hipGetErrorString(e));
-    } else {
-        rc = drain(ctx, (size_t)ctx->npts * rec, rec,
+    else
+        rc = stage_room(ctx, (size_t)ctx->npts * rec, rec, stage);
+    if (rc == AWP_OK) {
+        rc = drain(ctx, stage, (size_t)ctx->npts * rec, rec,
                    [ctx](int, size_t off, size_t, const void **src) {
                        *src = (const char *)ctx->d_sgt + off;
                        return AWP_OK;
@@ -1472,15 +1521,16 @@ extern "C" int awp_write_sgt_file_rwg(awp_ctx *ctx, const char *path, int zsourc
     float *d_out = nullptr;
     int *d_keep = nullptr;
     hipError_t e = hipSetDevice(ctx->device);
-    int rc = e == hipSuccess ? drain_room(ctx, unit) : AWP_OK;
-    if (rc == AWP_OK && e == hipSuccess) e = hipMalloc((void **)&d_out, 2 * ctx->pin_half);
+    Stage stage;
+    int rc = e == hipSuccess ? stage_room(ctx, nrec * unit, unit, stage) : AWP_OK;
+    if (rc == AWP_OK && e == hipSuccess) e = hipMalloc((void **)&d_out, (stage.pinned ? 2 : 1) * stage.half);
     if (rc == AWP_OK && e == hipSuccess) e = hipMalloc((void **)&d_keep, std::max<size_t>(nrec, 1) * sizeof(int));
     if (rc == AWP_OK && e == hipSuccess && nrec)
         e = hipMemcpy(d_keep, ctx->keep.data(), nrec * sizeof(int), hipMemcpyHostToDevice);
     if (rc == AWP_OK && e == hipSuccess)
-        rc = drain(ctx, nrec * unit, unit,
+        rc = drain(ctx, stage, nrec * unit, unit,
                    [&](int h, size_t off, size_t n, const void **src) -> int {
-                       float *out = (float *)((char *)d_out + (size_t)h * ctx->pin_half);
+                       float *out = (float *)((char *)d_out + (size_t)h * stage.half);
                        *src = out;
                        const size_t g0 = off / unit;
                        HIPTRY(ctx, launch_sgt_rwg(ctx->d_sgt, d_keep + g0, (int)g0, (int)(n / unit), ctx->nsamp_max,
@@ -1551,8 +1601,10 @@ extern "C" int awp_write_sgt_file_fp16(awp_ctx *ctx, const char *path)
         const void *dev;
         size_t bytes;
     } piece[2] = {{d_scale, npts * 6 * sizeof(float)}, {d_data, npts * 6 * (size_t)nsamp * sizeof(uint16_t)}};
+    Stage stage;
+    if (rc == AWP_OK) rc = stage_room(ctx, std::max(piece[0].bytes, piece[1].bytes), 64, stage);
     for (int q = 0; q < 2 && rc == AWP_OK; ++q) {
-        rc = drain(ctx, piece[q].bytes, 64,
+        rc = drain(ctx, stage, piece[q].bytes, 64,
                    [&](int, size_t off, size_t, const void **src) {
                        *src = (const char *)piece[q].dev + off;
                        return AWP_OK;

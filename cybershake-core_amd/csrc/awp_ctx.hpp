@@ -67,7 +67,7 @@ struct awp_ctx {
     float *d_sg;
     float *d_sgt;            // [npts][6][nsamp_max]
     std::vector<int> keep;   // per cordfile point
-    // pinned staging of the SGT output (drain): two halves of pin_half bytes,
+    // pinned staging of the SGT output (Stage): two halves of pin_half bytes,
     // made on the first large read and kept for the next
     char *pin;
     size_t pin_half;

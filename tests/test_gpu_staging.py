@@ -1,0 +1,111 @@
+"""How SGT output reaches the host: through pinned memory where there is any,
+through pageable memory where it is refused.  A child process whose
+hipHostMalloc goes through a counting stand-in, which can refuse, checks that
+every reader and writer gives the same bytes both ways."""
+import os
+import subprocess
+import sys
+
+import numpy as np
+import pytest
+
+import awpsgt
+import cases
+from conftest import REPO
+
+pytestmark = pytest.mark.gpu
+
+SHIM = r"""
+#include <dlfcn.h>
+#include <stddef.h>
+static int refuse, calls;
+static int (*real)(void **, size_t, unsigned);
+int shim_open(const char *lib)
+{
+    void *h = dlopen(lib, RTLD_LAZY | RTLD_NOLOAD);
+    real = h ? (int (*)(void **, size_t, unsigned))dlsym(h, "hipHostMalloc") : NULL;
+    return real != NULL;
+}
+void shim_refuse(int on) { refuse = on; }
+int shim_calls(void) { return calls; }
+int hipHostMalloc(void **p, size_t n, unsigned flags)
+{
+    ++calls;
+    return refuse || !real ? 2 : real(p, n, flags);   /* 2: hipErrorOutOfMemory */
+}
+"""
+
+CHILD = r"""
+import ctypes, os, sys
+shim = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)   # before the library that calls it
+for p in (%r, %r, %r, %r):
+    sys.path.insert(0, p)
+import numpy as np
+import awpsgt
+from test_gpu_parity import _inputs
+
+awpsgt.lib()
+hip = [ln.split()[-1] for ln in open("/proc/self/maps") if "libamdhip64" in ln][0]
+assert shim.shim_open(hip.encode())
+
+def make(d):
+    p, media, xyz, stf, pts = _inputs(d)
+    r = awpsgt.Run(p)
+    r.set_media(media)
+    r.set_source(xyz, stf)
+    r.set_sgt_points(pts)
+    r.init()
+    r.step(r.p.nt)
+    r.synchronize()
+    return r
+
+def outputs(r, d):
+    out = [r.sgt().tobytes()]
+    for name, write in (("raw", r.write_sgt_file), ("rwg", lambda f: r.write_sgt_file_rwg(f, True)),
+                        ("half", r.write_sgt_file_fp16)):
+        f = os.path.join(d, name)
+        write(f)
+        out.append(open(f, "rb").read())
+    return out
+"""
+
+
+def _child(tmp_path, body, *args):
+    src, lib = os.path.join(str(tmp_path), "shim.c"), os.path.join(str(tmp_path), "shim.so")
+    open(src, "w").write(SHIM)
+    subprocess.run(["gcc", "-shared", "-fPIC", "-O1", "-o", lib, src, "-ldl"], check=True)
+    here = [REPO, os.path.join(REPO, "cybershake-core_amd"), os.path.join(REPO, "tests", "golden"),
+            os.path.join(REPO, "tests")]
+    r = subprocess.run([sys.executable, "-c", CHILD % tuple(here) + body, lib] + list(args), stdout=subprocess.PIPE,
+                       stderr=subprocess.STDOUT, text=True, timeout=100)
+    assert r.returncode == 0, r.stdout
+    return r.stdout
+
+
+def _case(d, npts):
+    spec = cases.RunSpec(nx=48, ny=40, nz=32, dh=200.0, dt=0.01, nt=45, igreen=3, src=(24, 20, 4), nd=8, sigma=0.03,
+                         t0=0.12, ntiskp_sgt=1, write_step=20)
+    media = awpsgt.inputs.layered_media(48, 40, 32, [700.0, 1500.0, 2500.0])
+    rng = np.random.default_rng(6)
+    pts = np.stack([rng.integers(1, m + 1, npts) for m in (48, 40, 32)], -1)
+    pts[[0, npts // 3, npts - 1], 0] = 49      # dropped
+    cases.write_case(d, spec, media, pts)
+    return d
+
+
+def test_pinned_memory_refused(tmp_path):
+    """77 MB of output: every call falls back to pageable memory, and a
+    later run of the process takes pinned memory again."""
+    d = _case(str(tmp_path), 72000)
+    _child(tmp_path, r"""
+shim.shim_refuse(1)
+r = make(sys.argv[2])
+a = outputs(r, sys.argv[2])
+n = shim.shim_calls()
+assert n >= 1
+shim.shim_refuse(0)
+q = make(sys.argv[2])
+b = outputs(q, sys.argv[2])
+assert shim.shim_calls() == n + 1      # one buffer, kept for the run's later reads
+assert a == b and len(a[0]) == 72000 * 6 * 45 * 4 and any(a[0])
+""", d)
