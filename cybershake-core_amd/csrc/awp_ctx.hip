@@ -1262,11 +1262,13 @@ extern "C" int awp_device_bytes(const awp_ctx *ctx, size_t *bytes)
 namespace {
 
 // The host memory one transfer of SGT output goes through: the run's pinned
-// buffer (two halves), or, where pinned memory is refused, pageable memory of
+// buffer (two halves), which one transfer holds at a time, or, where another
+// thread's transfer holds it or pinned memory is refused, pageable memory of
 // the transfer's own (one half).
 constexpr size_t PIN_HALF = (size_t)16 << 20;
 
 struct Stage {
+    std::unique_lock<std::mutex> lock;   // on the run's pinned buffer and its events
     char *host = nullptr;
     size_t half = 0;
     bool pinned = false;
@@ -1279,9 +1281,11 @@ struct Stage {
     }
 };
 
-// the pinned buffer, if there is one whose halves hold a unit
+// the pinned buffer, if it is free and its halves hold a unit
 void pin_room(awp_ctx *ctx, size_t unit, Stage &s)
 {
+    s.lock = std::unique_lock<std::mutex>(ctx->pin_busy, std::try_to_lock);
+    if (!s.lock.owns_lock()) return;
     if (!ctx->pin) {
         const size_t half = std::max(PIN_HALF, unit);
         char *p = nullptr;

@@ -9,6 +9,7 @@
 #include <stdio.h>
 #include <string.h>
 
+#include <mutex>
 #include <vector>
 
 #include "awp_kernels.hpp"
@@ -68,7 +69,9 @@ struct awp_ctx {
     float *d_sgt;            // [npts][6][nsamp_max]
     std::vector<int> keep;   // per cordfile point
     // pinned staging of the SGT output (Stage): two halves of pin_half bytes,
-    // made on the first large read and kept for the next
+    // made on the first large read and kept for the next; pin_busy: held by the
+    // transfer that uses them
+    std::mutex pin_busy;
     char *pin;
     size_t pin_half;
     hipEvent_t pin_ev[2];

@@ -109,3 +109,37 @@ b = outputs(q, sys.argv[2])
 assert shim.shim_calls() == n + 1      # one buffer, kept for the run's later reads
 assert a == b and len(a[0]) == 72000 * 6 * 45 * 4 and any(a[0])
 """, d)
+
+
+def test_threads_share_a_run(tmp_path):
+    """Four threads read and write one finished run at the same time, more
+    than once: each gets the bytes a thread alone gets."""
+    from concurrent.futures import ThreadPoolExecutor
+    from test_gpu_batch import _make
+    d = _case(str(tmp_path), 36000)
+    r = _make(d, awpsgt.AWP_STORAGE_FP32)
+    r.step(r.p.nt)
+    r.synchronize()
+
+    def job(kind, n):
+        f = os.path.join(d, "%s%d" % (kind, n))
+        if kind == "sgt":
+            return r.sgt().tobytes()
+        if kind == "rwg":
+            r.write_sgt_file_rwg(f)
+        else:
+            (r.write_sgt_file if kind == "raw" else r.write_sgt_file_fp16)(f)
+        return open(f, "rb").read()
+
+    kinds = ["sgt", "raw", "rwg", "half"]
+    want = {k: job(k, 99) for k in kinds}
+    q = _make(d, awpsgt.AWP_STORAGE_FP32)      # a run that has made no buffer yet
+    q.step(q.p.nt)
+    q.synchronize()
+    for x in (r, q):
+        r = x
+        with ThreadPoolExecutor(4) as ex:
+            got = list(ex.map(lambda n: (kinds[n % 4], job(kinds[n % 4], n)), range(16)))
+        for k, b in got:
+            assert b == want[k], k
+        x.close()
