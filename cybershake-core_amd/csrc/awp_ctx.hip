@@ -1383,6 +1383,9 @@ void parts(size_t n, size_t bytes, FN fn)
     }, &arg);
 }
 
+// One thread writes: a file takes one write at a time (its inode's lock), and
+// eight threads that wait for it in turn took 17 ms for a 77 MB RWG file and
+// 37 for 154 MB, where one takes 10.6 and 20.4.
 bool write_at(int fd, const char *p, size_t n, off_t off)
 {
     while (n) {
@@ -1542,11 +1545,7 @@ extern "C" int awp_write_sgt_file_rwg(awp_ctx *ctx, const char *path, int zsourc
                        return AWP_OK;
                    },
                    [&](const char *h, size_t off, size_t m) {
-                       std::atomic<bool> ok(true);
-                       parts(m / unit, m, [&](size_t a, size_t b) {
-                           if (!write_at(fd, h + a * unit, (b - a) * unit, (off_t)(off + a * unit))) ok = false;
-                       });
-                       return ok ? AWP_OK : fail(ctx, AWP_EIO, "write '%s' failed", path);
+                       return write_at(fd, h, m, (off_t)off) ? AWP_OK : fail(ctx, AWP_EIO, "write '%s' failed", path);
                    });
     hipFree(d_out);
     hipFree(d_keep);
@@ -1614,11 +1613,8 @@ extern "C" int awp_write_sgt_file_fp16(awp_ctx *ctx, const char *path)
                        return AWP_OK;
                    },
                    [&](const char *h, size_t off, size_t m) {
-                       std::atomic<bool> ok(true);
-                       parts(m, m, [&](size_t a, size_t b) {
-                           if (!write_at(fd, h + a, b - a, (off_t)(base + off + a))) ok = false;
-                       });
-                       return ok ? AWP_OK : fail(ctx, AWP_EIO, "write '%s' failed", path);
+                       return write_at(fd, h, m, (off_t)(base + off)) ? AWP_OK
+                                                                      : fail(ctx, AWP_EIO, "write '%s' failed", path);
                    });
         base += piece[q].bytes;
     }
