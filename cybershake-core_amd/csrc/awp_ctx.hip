@@ -377,7 +377,7 @@ extern "C" int awp_create(awp_ctx **out, const awp_in3d *p, int device, int stor
     ctx->d_trace = nullptr;
     ctx->trace_pos = 0;
     ctx->pin = nullptr;
-    ctx->pin_half = 0;
+    ctx->pin_half = ctx->moved = 0;
     ctx->pin_ev[0] = ctx->pin_ev[1] = nullptr;
 
     e = hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking);
@@ -1261,11 +1261,33 @@ extern "C" int awp_device_bytes(const awp_ctx *ctx, size_t *bytes)
 // ---------------------------------------------------------------------------
 namespace {
 
+// fn(a, b) over parts [a, b) of n items, on as many threads as `bytes` of
+// copying are worth
+template <class FN>
+void parts(size_t n, size_t bytes, FN fn)
+{
+    struct Arg {
+        size_t n;
+        FN *fn;
+    } arg = {n, &fn};
+    const int np = (int)std::min<size_t>(awp_par_threads(bytes), std::max<size_t>(n, 1));
+    awp_par(np, [](void *p, int k, int m) {
+        Arg *a = (Arg *)p;
+        (*a->fn)(a->n * (size_t)k / (size_t)m, a->n * (size_t)(k + 1) / (size_t)m);
+    }, &arg);
+}
+
 // The host memory one transfer of SGT output goes through: the run's pinned
 // buffer (two halves), which one transfer holds at a time, or, where another
 // thread's transfer holds it or pinned memory is refused, pageable memory of
-// the transfer's own (one half).
+// the transfer's own.
 constexpr size_t PIN_HALF = (size_t)16 << 20;
+// The buffer is made once a run's transfers add up to PIN_FROM bytes.  Its
+// pages cost 1.5 us each on the host's first access, 12 ms in all (2.4 by eight
+// threads): more than it saves a run that is read once.  First sgt() of a run,
+// pageable / pinned: 19 MB 1.1 / 2.9 ms, 38 MB 3.7 / 1.4-4.2, 77 MB 7.4 /
+// 2.7-5.0; first FP16 file of 0.5 MB 0.13 / 0.62.
+constexpr size_t PIN_FROM = (size_t)64 << 20;
 
 struct Stage {
     std::unique_lock<std::mutex> lock;   // on the run's pinned buffer and its events
@@ -1281,12 +1303,15 @@ struct Stage {
     }
 };
 
-// the pinned buffer, if it is free and its halves hold a unit
-void pin_room(awp_ctx *ctx, size_t unit, Stage &s)
+// the pinned buffer for a transfer of `bytes`, if it is free, its halves hold
+// a unit and the run has moved enough to have one
+void pin_room(awp_ctx *ctx, size_t bytes, size_t unit, Stage &s)
 {
-    s.lock = std::unique_lock<std::mutex>(ctx->pin_busy, std::try_to_lock);
-    if (!s.lock.owns_lock()) return;
+    std::unique_lock<std::mutex> lock(ctx->pin_busy, std::try_to_lock);
+    if (!lock.owns_lock()) return;
+    ctx->moved += bytes;
     if (!ctx->pin) {
+        if (ctx->moved < PIN_FROM) return;
         const size_t half = std::max(PIN_HALF, unit);
         char *p = nullptr;
         bool ok = true;
@@ -1297,10 +1322,15 @@ void pin_room(awp_ctx *ctx, size_t unit, Stage &s)
             (void)hipGetLastError();   // not the next call's error
             return;
         }
+        const size_t page = 4096;
+        parts(2 * half / page, 2 * half, [=](size_t a, size_t b) {
+            for (size_t q = a; q < b; ++q) ((volatile char *)p)[q * page] = 0;
+        });
         ctx->pin = p;
         ctx->pin_half = half;
     }
     if (ctx->pin_half < unit) return;
+    s.lock = std::move(lock);
     s.host = ctx->pin;
     s.half = ctx->pin_half;
     s.pinned = true;
@@ -1309,7 +1339,7 @@ void pin_room(awp_ctx *ctx, size_t unit, Stage &s)
 // staging of a transfer of `bytes` in whole units
 int stage_room(awp_ctx *ctx, size_t bytes, size_t unit, Stage &s)
 {
-    pin_room(ctx, unit, s);
+    pin_room(ctx, bytes, unit, s);
     if (s.pinned) return AWP_OK;
     s.half = std::max(std::min(PIN_HALF, bytes), unit);
     s.host = (char *)malloc(s.half);
@@ -1367,22 +1397,6 @@ int drain(awp_ctx *ctx, const Stage &s, size_t bytes, size_t unit, MAKE make, US
     return AWP_OK;
 }
 
-// fn(a, b) over parts [a, b) of n items, on as many threads as `bytes` of
-// copying are worth
-template <class FN>
-void parts(size_t n, size_t bytes, FN fn)
-{
-    struct Arg {
-        size_t n;
-        FN *fn;
-    } arg = {n, &fn};
-    const int np = (int)std::min<size_t>(awp_par_threads(bytes), std::max<size_t>(n, 1));
-    awp_par(np, [](void *p, int k, int m) {
-        Arg *a = (Arg *)p;
-        (*a->fn)(a->n * (size_t)k / (size_t)m, a->n * (size_t)(k + 1) / (size_t)m);
-    }, &arg);
-}
-
 // One thread writes: a file takes one write at a time (its inode's lock), and
 // eight threads that wait for it in turn took 17 ms for a 77 MB RWG file and
 // 37 for 154 MB, where one takes 10.6 and 20.4.
@@ -1408,7 +1422,7 @@ extern "C" int awp_get_sgt(awp_ctx *ctx, float *host, size_t count)
     if (count < n) return fail(ctx, AWP_EINVAL, "buffer holds %zu floats, need %zu", count, n);
     HIPTRY(ctx, hipSetDevice(ctx->device));
     Stage stage;
-    if (n * sizeof(float) >= ((size_t)8 << 20)) pin_room(ctx, 64, stage);
+    if (n * sizeof(float) >= ((size_t)8 << 20)) pin_room(ctx, n * sizeof(float), 64, stage);
     if (!stage.pinned) {
         HIPTRY(ctx, hipStreamSynchronize(ctx->stream));
         if (n) HIPTRY(ctx, hipMemcpy(host, ctx->d_sgt, n * sizeof(float), hipMemcpyDeviceToHost));
@@ -1605,7 +1619,7 @@ extern "C" int awp_write_sgt_file_fp16(awp_ctx *ctx, const char *path)
         size_t bytes;
     } piece[2] = {{d_scale, npts * 6 * sizeof(float)}, {d_data, npts * 6 * (size_t)nsamp * sizeof(uint16_t)}};
     Stage stage;
-    if (rc == AWP_OK) rc = stage_room(ctx, std::max(piece[0].bytes, piece[1].bytes), 64, stage);
+    if (rc == AWP_OK) rc = stage_room(ctx, piece[0].bytes + piece[1].bytes, 64, stage);
     for (int q = 0; q < 2 && rc == AWP_OK; ++q) {
         rc = drain(ctx, stage, piece[q].bytes, 64,
                    [&](int, size_t off, size_t, const void **src) {

@@ -69,11 +69,11 @@ struct awp_ctx {
     float *d_sgt;            // [npts][6][nsamp_max]
     std::vector<int> keep;   // per cordfile point
     // pinned staging of the SGT output (Stage): two halves of pin_half bytes,
-    // made on the first large read and kept for the next; pin_busy: held by the
-    // transfer that uses them
+    // made when the run's transfers so far (moved, bytes) are worth it and kept
+    // for the next; pin_busy: held by the transfer that uses them
     std::mutex pin_busy;
     char *pin;
-    size_t pin_half;
+    size_t pin_half, moved;
     hipEvent_t pin_ev[2];
     // progress
     bool media_set, source_set, points_set, initialised;

@@ -143,3 +143,21 @@ def test_threads_share_a_run(tmp_path):
         for k, b in got:
             assert b == want[k], k
         x.close()
+
+
+def test_small_output_makes_no_pinned_buffer(tmp_path):
+    """A run whose output is read once, 2 to 26 MB of it, makes no pinned
+    buffer (which costs more than it saves there); one that reads 64 MB in
+    all makes one, once."""
+    small, large = (_case(os.path.join(str(tmp_path), n), k) for n, k in (("small", 2000), ("large", 24000)))
+    _child(tmp_path, r"""
+r = make(sys.argv[2])
+a = outputs(r, sys.argv[2])
+assert len(a[0]) == 2000 * 6 * 45 * 4 and shim.shim_calls() == 0
+r = make(sys.argv[3])
+a = [r.sgt() for k in range(2)]
+assert a[0].nbytes == 24000 * 6 * 45 * 4 and shim.shim_calls() == 0
+a += [r.sgt() for k in range(3)]
+assert shim.shim_calls() == 1
+assert all(np.array_equal(a[0], b) for b in a) and np.any(a[0] != 0)
+""", small, large)
