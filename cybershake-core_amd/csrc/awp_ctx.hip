@@ -4,6 +4,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <errno.h>
 #include <fcntl.h>
 #include <math.h>
 #include <stdarg.h>
@@ -1397,16 +1398,31 @@ int drain(awp_ctx *ctx, const Stage &s, size_t bytes, size_t unit, MAKE make, US
     return AWP_OK;
 }
 
-// One thread writes: a file takes one write at a time (its inode's lock), and
-// eight threads that wait for it in turn took 17 ms for a 77 MB RWG file and
-// 37 for 154 MB, where one takes 10.6 and 20.4.
+// n bytes at off of fd, or false
 bool write_at(int fd, const char *p, size_t n, off_t off)
 {
     while (n) {
         const ssize_t w = pwrite(fd, p, n, off);
+        if (w < 0 && errno == EINTR) continue;
         if (w <= 0) return false;
         p += w;
         off += w;
+        n -= (size_t)w;
+    }
+    return true;
+}
+
+// A file written from its start to its end; also a pipe or another target
+// that cannot seek.  By one thread: a file takes one write at a time (its
+// inode's lock), and eight threads that wait for it in turn took 17 ms for a
+// 77 MB RWG file and 37 for 154 MB, where one takes 10.6 and 20.4.
+bool append(int fd, const char *p, size_t n)
+{
+    while (n) {
+        const ssize_t w = write(fd, p, n);
+        if (w < 0 && errno == EINTR) continue;
+        if (w <= 0) return false;
+        p += w;
         n -= (size_t)w;
     }
     return true;
@@ -1558,8 +1574,8 @@ extern "C" int awp_write_sgt_file_rwg(awp_ctx *ctx, const char *path, int zsourc
                                                   nt_out, navail, zsource ? 1 : 0, out, ctx->stream));
                        return AWP_OK;
                    },
-                   [&](const char *h, size_t off, size_t m) {
-                       return write_at(fd, h, m, (off_t)off) ? AWP_OK : fail(ctx, AWP_EIO, "write '%s' failed", path);
+                   [&](const char *h, size_t, size_t m) {
+                       return append(fd, h, m) ? AWP_OK : fail(ctx, AWP_EIO, "write '%s' failed", path);
                    });
     hipFree(d_out);
     hipFree(d_keep);
@@ -1611,9 +1627,8 @@ extern "C" int awp_write_sgt_file_fp16(awp_ctx *ctx, const char *path)
     memcpy(hdr + 32, &nto, 4);
     int fd = open(path, O_WRONLY | O_CREAT | O_TRUNC, 0666);
     int rc = fd < 0 ? fail(ctx, AWP_EIO, "cannot create '%s'", path)
-                    : write_at(fd, (const char *)hdr, 64, 0) ? AWP_OK : fail(ctx, AWP_EIO, "write '%s' failed", path);
+                    : append(fd, (const char *)hdr, 64) ? AWP_OK : fail(ctx, AWP_EIO, "write '%s' failed", path);
     // the header, then the scales, then the series
-    size_t base = 64;
     const struct {
         const void *dev;
         size_t bytes;
@@ -1626,11 +1641,9 @@ extern "C" int awp_write_sgt_file_fp16(awp_ctx *ctx, const char *path)
                        *src = (const char *)piece[q].dev + off;
                        return AWP_OK;
                    },
-                   [&](const char *h, size_t off, size_t m) {
-                       return write_at(fd, h, m, (off_t)(base + off)) ? AWP_OK
-                                                                      : fail(ctx, AWP_EIO, "write '%s' failed", path);
+                   [&](const char *h, size_t, size_t m) {
+                       return append(fd, h, m) ? AWP_OK : fail(ctx, AWP_EIO, "write '%s' failed", path);
                    });
-        base += piece[q].bytes;
     }
     hipStreamSynchronize(ctx->stream);
     hipFree(d_scale);

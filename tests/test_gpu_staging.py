@@ -161,3 +161,26 @@ a += [r.sgt() for k in range(3)]
 assert shim.shim_calls() == 1
 assert all(np.array_equal(a[0], b) for b in a) and np.any(a[0] != 0)
 """, small, large)
+
+
+def test_writers_into_a_pipe(tmp_path):
+    """The RWG-order and FP16 writers go from start to end, so a pipe takes
+    them: the same bytes as the file."""
+    import threading
+    from test_gpu_batch import _make
+    d = _case(str(tmp_path), 9000)
+    r = _make(d, awpsgt.AWP_STORAGE_FP32)
+    r.step(r.p.nt)
+    r.synchronize()
+    for n, write in enumerate((r.write_sgt_file_rwg, lambda f: r.write_sgt_file_rwg(f, True), r.write_sgt_file_fp16)):
+        plain, pipe = (os.path.join(d, "%s%d" % (k, n)) for k in ("plain", "pipe"))
+        write(plain)
+        os.mkfifo(pipe)
+        got = []
+        t = threading.Thread(target=lambda: got.append(open(pipe, "rb").read()), daemon=True)
+        t.start()
+        write(pipe)
+        t.join(20)
+        want = open(plain, "rb").read()
+        assert got and got[0] == want and len(want) > 1000000
+    r.close()
