@@ -296,12 +296,13 @@ extern "C" int awp_batch_create(awp_batch **out, awp_ctx *const *runs, int nruns
     b->claims = !(ce && !strcmp(ce, "0"));
     b->o32 = true;
     for (int r = 0; r < nruns; ++r) b->o32 = b->o32 && runs[r]->l.o32;
-    b->l = runs[0]->l;
+    // run 0's launch shape, or the batch scheme's default for it where it steps
+    // by the other one
+    b->l = runs[0]->fused != b->split ? runs[0]->l : choose_launch(runs[0]->g, !b->split, b->mixed, b->device);
     if (b->split) {
         // two-stage kernels: {64, 128} x {1, 2, 4, 8} tiles, z unroll 1 or 2;
         // blocks of more than 512 threads (64 x 16, 128 x 8) in the
         // byte-offset stress form without z unroll
-        if (runs[0]->fused) b->l.tile_y = 4;   // a fused run's launch shape is no guide
         if (b->l.unroll != 2) b->l.unroll = 1;
         if (b->l.tile_xw != 2) b->l.tile_xw = 1;
         const bool tall_ok = b->o32 && b->l.o32_s && b->l.unroll == 1;
@@ -323,7 +324,6 @@ extern "C" int awp_batch_create(awp_batch **out, awp_ctx *const *runs, int nruns
         for (int r = 0; r < nruns; ++r) nvol += runs[r]->g.nvol;
         if (b->split && nruns > 1) b->l.cached = cache_mode(nvol, b->mixed);
         b->l.o32 = b->o32;
-        if (runs[0]->fused) b->l.claim = 0;   // a fused run's claims
         if (b->split && !b->persist)
             choose_staged(b->l, b->mixed);
         else

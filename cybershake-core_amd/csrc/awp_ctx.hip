@@ -167,7 +167,7 @@ static void set_chunks(Launch &l, const Geo &g, int nchunk, bool fused)
     l.nchunk = (g.nz + l.kc - 1) / l.kc;
 }
 
-static Launch choose_launch(const Geo &g, bool fused, bool mixed, int device)
+Launch choose_launch(const Geo &g, bool fused, bool mixed, int device)
 {
     Launch l;
     // two-stage: 64 x 4 tiles, 64 x 2 where the chunks are short (split_kc).

@@ -105,6 +105,9 @@ struct awp_ctx {
     }
 };
 
+// the default launch shape of a run of these sizes by either scheme
+Launch choose_launch(const Geo &g, bool fused, bool mixed, int device);
+
 inline int fail(awp_ctx *ctx, int code, const char *fmt, ...)
 {
     if (ctx) {

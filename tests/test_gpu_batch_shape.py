@@ -1,0 +1,54 @@
+"""The scheme and launch shape a batch takes from its runs."""
+import numpy as np
+import pytest
+
+import awpsgt
+from test_gpu_batch import _make
+from test_gpu_staged import _case, _equal
+
+pytestmark = pytest.mark.gpu
+
+
+def _runs(tmp_path, sizes, storage=awpsgt.AWP_STORAGE_FP32):
+    return [_make(_case(tmp_path / str(n), *q, 1 + n % 3, (q[0] // 2, q[1] // 2, 5)), storage)
+            for n, q in enumerate(sizes)]
+
+
+def test_fused_batch_of_two_stage_runs(tmp_path, monkeypatch):
+    """Small FP32 runs step two-stage by themselves; a fused batch of them
+    takes the fused step's default shape, not their two-stage tiles."""
+    runs, refs = (_runs(tmp_path, [(70, 34, 40), (48, 40, 32), (130, 25, 24)]) for _ in range(2))
+    assert not any(r.scheme()[0] for r in runs)
+    monkeypatch.setenv("AWP_BATCH_SCHEME", "fused")
+    with awpsgt.Batch(runs) as b:
+        assert b.fused() and b.launch()[:2] == (11, 3)
+        b.step(6)
+        b.step(runs[0].p.nt)
+    for r, ref in zip(runs, refs):
+        ref.step(ref.p.nt)
+        ref.synchronize()
+        _equal(ref, r)
+        r.close()
+        ref.close()
+
+
+@pytest.mark.parametrize("storage", [awpsgt.AWP_STORAGE_FP32, awpsgt.AWP_STORAGE_MIXED])
+def test_two_stage_batch_of_fused_runs(storage, tmp_path, monkeypatch):
+    """The other way round: the shape a two-stage run of the sizes has."""
+    sizes = [(70, 34, 40), (48, 40, 32), (130, 25, 24)]
+    monkeypatch.setenv("AWP_SCHEME", "split")
+    refs = _runs(tmp_path, sizes, storage)
+    with awpsgt.Batch(refs) as b:
+        want = b.launch()
+        b.step(refs[0].p.nt)
+    monkeypatch.setenv("AWP_SCHEME", "fused")
+    runs = _runs(tmp_path, sizes, storage)
+    monkeypatch.setenv("AWP_BATCH_SCHEME", "split")
+    with awpsgt.Batch(runs) as b:
+        assert not b.fused() and b.launch() == want
+        b.step(7)
+        b.step(runs[0].p.nt)
+    for r, ref in zip(runs, refs):
+        _equal(ref, r)
+        r.close()
+        ref.close()
