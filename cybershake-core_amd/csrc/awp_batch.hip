@@ -276,14 +276,24 @@ extern "C" int awp_batch_create(awp_batch **out, awp_ctx *const *runs, int nruns
     b->runs.assign(runs, runs + nruns);
     b->device = runs[0]->device;
     b->mixed = runs[0]->mixed();
-    // the fused scheme when every run holds both buffers and steps fused
+    // The fused scheme when every run holds both buffers and steps fused, or
+    // steps two-stage by its own size alone and the batch has FUSED_POINTS.  us
+    // per step, two-stage / fused: 3 x 131x97x53 (2M) 94 / 115, 16 x 131x97x53
+    // (11M) 503 / 540, 4 x 200x200x100 (16M) 592 / 635, 2 x 320x320x128 (26M)
+    // 940 / 919, 40 x 131x97x53 (27M) 1263 / 1188, 8 x 200x200x100 1349 / 1245, 3
+    // x 300x300x120 1100 / 1030, 400x300x150 with 733x566x196 3662 / 3240,
+    // 200x200x100 with 1500x1000x300 15290 / 13980.
     b->can_fuse = true;
-    bool all_fused = true;
+    bool all_fused = true, open = true;
+    long long points = 0;
     for (int r = 0; r < nruns; ++r) {
-        b->can_fuse = b->can_fuse && runs[r]->two_bufs;
-        all_fused = all_fused && runs[r]->fused;
+        const awp_ctx *c = runs[r];
+        b->can_fuse = b->can_fuse && c->two_bufs;
+        all_fused = all_fused && c->fused;
+        open = open && (c->fused || c->by_size);
+        points += (long long)c->g.nx * c->g.ny * c->g.nz;
     }
-    b->split = !(b->can_fuse && all_fused);
+    b->split = !(b->can_fuse && (all_fused || (open && points >= FUSED_POINTS)));
     // AWP_BATCH_SCHEME=fused / split overrides (fused only where every run
     // holds both buffers; each run's own step is unchanged)
     const char *bs = getenv("AWP_BATCH_SCHEME");

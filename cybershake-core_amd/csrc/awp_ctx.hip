@@ -129,15 +129,18 @@ static bool want_fused(const Geo &g, int storage)
 }
 
 // Whether a run that holds both buffers starts on the fused step: always
-// under AWP_SCHEME=fused, else from 25M points on (below, a tile a CU leaves
+// under AWP_SCHEME=fused, else from FUSED_POINTS on (below, a tile a CU leaves
 // too few rounds to even out).  FP32, two-stage against fused on the same
-// buffers, us per step: 200x200x100 165 against 196, 300x300x120 414 against
-// 428, 517x389x149 (30M) 1133 against 1101, 800x600x200 3430 against 3193,
-// 1500x1000x300 16290 against 14640.
+// buffers, us per step: 200x200x100 165 against 196, 256x256x128 (8M) 311 / 320,
+// 300x300x120 414 / 428, 320x320x128 (13M) 473 / 474, 400x300x150 (18M) 676 /
+// 671, 448x320x160 (23M) 828 / 805, 1000x250x100 (25M) 907 / 874, 700x600x64
+// (27M) 1009 / 951, 300x300x300 1063 / 974, 517x389x149 (30M) 1133 / 1101,
+// 1500x100x200 1099 / 992, 1024x1024x32 (34M) 1161 / 1161, 800x600x200 3430 /
+// 3193, 1500x1000x300 16290 / 14640.
 static bool start_fused(const Geo &g)
 {
     const char *scheme = getenv("AWP_SCHEME");
-    return (scheme && !strcmp(scheme, "fused")) || (long long)g.nx * g.ny * g.nz >= 25000000ll;
+    return (scheme && !strcmp(scheme, "fused")) || (long long)g.nx * g.ny * g.nz >= FUSED_POINTS;
 }
 
 // z chunks of `nchunk` requested: the top chunk keeps >= 3 levels (the
@@ -350,6 +353,7 @@ extern "C" int awp_create(awp_ctx **out, const awp_in3d *p, int device, int stor
     ctx->g = make_geo(p->nx, p->ny, p->nz);
     ctx->two_bufs = want_fused(ctx->g, storage);
     ctx->fused = ctx->two_bufs && start_fused(ctx->g);
+    ctx->by_size = true;
     ctx->l = choose_launch(ctx->g, ctx->fused, storage == AWP_STORAGE_MIXED, device);
     ctx->vol = nullptr;
     ctx->prof = nullptr;
@@ -1015,6 +1019,7 @@ extern "C" int awp_set_scheme(awp_ctx *ctx, int fused)
     HIPTRY(ctx, hipSetDevice(ctx->device));
     HIPTRY(ctx, hipStreamSynchronize(ctx->stream));
     ctx->fused = fused != 0;
+    ctx->by_size = false;
     ctx->l = choose_launch(ctx->g, ctx->fused, ctx->mixed(), ctx->device);
     return scheme_changed(ctx);
 }
@@ -1175,6 +1180,7 @@ extern "C" int awp_tune(awp_ctx *ctx, int reps)
     };
     rc = search();
     if (rc) return rc;
+    ctx->by_size = false;
     // the trial steps changed the state: start the run again
     return awp_init(ctx);
 }

@@ -21,6 +21,10 @@ using awp::Launch;
 using awp::Media32;
 using awp::State;
 
+// points from which the fused step of an FP32 run or batch is the faster one
+// (start_fused, awp_batch_create)
+constexpr long long FUSED_POINTS = 25000000;
+
 struct awp_ctx {
     awp_in3d p;
     int device;
@@ -36,6 +40,7 @@ struct awp_ctx {
     float *wf[2][9];
     int cur;
     bool fused;              // the step in use: fused one-sweep (true) or two-stage
+    bool by_size;            // `fused` is awp_create's choice (not awp_set_scheme's or awp_tune's)
     bool two_bufs;           // the allocation holds wf[1] (the fused step can run)
     // the two-stage step's job table (one entry: this run), uploaded by
     // awp_init, and its tile count

@@ -52,3 +52,28 @@ def test_two_stage_batch_of_fused_runs(storage, tmp_path, monkeypatch):
         _equal(ref, r)
         r.close()
         ref.close()
+
+
+def test_batch_scheme_by_all_runs_sizes(tmp_path, monkeypatch):
+    """FP32 runs too small to step fused by themselves make a fused batch
+    when they hold 25M points together; not below, and not where a run was
+    put on the two-stage step."""
+    sizes = [(300, 300, 100), (300, 280, 110), (250, 260, 120)]     # 9.0 + 9.24 + 7.8M
+    runs = _runs(tmp_path, sizes)
+    refs = _runs(tmp_path, sizes)
+    assert not any(r.scheme()[0] for r in runs)
+    with awpsgt.Batch(runs[:2]) as b:
+        assert not b.fused()
+    with awpsgt.Batch(runs) as b:
+        assert b.fused() and b.launch()[:2] == (11, 3)
+        b.step(7)
+    for r in refs:
+        r.set_scheme(False)
+    with awpsgt.Batch(refs) as b:
+        assert not b.fused()
+        b.step(7)
+    for r, ref in zip(runs, refs):
+        for f in ("u1", "xx", "yz", "r1", "r6"):
+            assert np.array_equal(r.field(f), ref.field(f)), f
+        r.close()
+        ref.close()
