@@ -112,6 +112,38 @@ static Launch run_launch(const Geo &g, const Launch &bl, int nchunk, bool split)
     return l;
 }
 
+// Default z chunks of the batch: the chain of a wave's levels is hidden by
+// every run's waves together.
+static int max_nz(const awp_batch *b)
+{
+    int nz = 0;
+    for (const awp_ctx *c : b->runs) nz = std::max(nz, c->g.nz);
+    return nz;
+}
+// chunks of each run in the FP32 fused step on 64 x 11 tiles
+static int sweep_chunks(const awp_batch *b)
+{
+    long long cols = 0;
+    for (const awp_ctx *c : b->runs) cols += (long long)((c->g.nx + TX - 1) / TX) * ((c->g.ny + 10) / 11);
+    return sweep_nchunk(cols, max_nz(b));
+}
+// levels a chunk of the two-stage kernels, staged and without LDS
+static int staged_levels(const awp_batch *b)
+{
+    long long cols = 0;
+    for (const awp_ctx *c : b->runs) cols += staged_cols(c->g);
+    const int nz = max_nz(b), n = staged_nchunk(cols, nz);
+    return (nz + n - 1) / n;
+}
+static int plain_levels(const awp_batch *b)
+{
+    long long rows = 0;
+    for (const awp_ctx *c : b->runs) rows += row_segments(c->g);
+    return split_kc(rows, max_nz(b));
+}
+// whether a fused shape runs awp_sweep.hpp
+static bool swept(const awp_batch *b, int tile_y, int unroll) { return !b->mixed && tile_y == 11 && unroll == 3; }
+
 // Builds the device job tables from the runs' current buffer parity: in the
 // fused scheme run r reads s[0] = its current state and writes s[1]; the
 // two-stage scheme updates the current state in place.
@@ -309,6 +341,7 @@ extern "C" int awp_batch_create(awp_batch **out, awp_ctx *const *runs, int nruns
     // run 0's launch shape, or the batch scheme's default for it where it steps
     // by the other one
     b->l = runs[0]->fused != b->split ? runs[0]->l : choose_launch(runs[0]->g, !b->split, b->mixed, b->device);
+    if (!b->split && !ce) b->l.claim = 0;   // a fused run's; no guide for the tuner's two-stage shapes
     if (b->split) {
         // two-stage kernels: {64, 128} x {1, 2, 4, 8} tiles, z unroll 1 or 2;
         // blocks of more than 512 threads (64 x 16, 128 x 8) in the
@@ -332,39 +365,15 @@ extern "C" int awp_batch_create(awp_batch **out, awp_ctx *const *runs, int nruns
         // the cache is shared by every run of a step
         long long nvol = 0;
         for (int r = 0; r < nruns; ++r) nvol += runs[r]->g.nvol;
-        if (b->split && nruns > 1) b->l.cached = cache_mode(nvol, b->mixed);
+        if (nruns > 1 || !b->split) b->l.cached = cache_mode(nvol, b->mixed);
         b->l.o32 = b->o32;
         if (b->split && !b->persist)
             choose_staged(b->l, b->mixed);
         else
             b->l.staged = false;
     }
-    b->nchunk.assign(nruns, 1);
-    // the chain of a wave's levels is hidden by every run's waves together
-    {
-        long long rows = 0;
-        int nz = 0;
-        for (int r = 0; r < nruns; ++r) {
-            rows += row_segments(runs[r]->g);
-            nz = std::max(nz, runs[r]->g.nz);
-        }
-        if (!b->split && !b->mixed && b->l.tile_y == 11 && b->l.unroll == 3) {
-            long long cols = 0;
-            for (int r = 0; r < nruns; ++r) {
-                const FTiles t = fused_tiles(runs[r]->g, b->l);
-                cols += (long long)t.nbx * t.nby;
-            }
-            b->nchunk.assign(nruns, sweep_nchunk(cols, nz));
-        }
-        if (b->l.staged) {
-            long long cols = 0;
-            for (int r = 0; r < nruns; ++r) cols += staged_cols(runs[r]->g);
-            const int n = staged_nchunk(cols, nz);
-            b->kc_split = (nz + n - 1) / n;
-        } else {
-            b->kc_split = split_kc(rows, nz);
-        }
-    }
+    b->nchunk.assign(nruns, !b->split && swept(b, b->l.tile_y, b->l.unroll) ? sweep_chunks(b) : 1);
+    b->kc_split = b->l.staged ? staged_levels(b) : plain_levels(b);
     b->d_jobs = nullptr;
     b->d_sjobs = nullptr;
     b->d_aux = nullptr;
@@ -500,22 +509,31 @@ extern "C" int awp_batch_tune(awp_batch *b, int reps)
     BTRY(b, hipSetDevice(b->device));
     struct Cand {
         bool split, persist;
-        int ty, pf, nchunk;   // nchunk: z chunks per run (fused), chunk length in levels (two-stage)
+        int ty, pf, nchunk;   // nchunk: z chunks per run (fused; 0 = sweep_chunks), chunk length in levels (two-stage)
         int xw;      // two-stage: waves per tile row
         int sform;   // two-stage stress kernel: 0 = 64-bit offsets, 1 = 32-bit offsets, 2 blocks per
                      // CU; 2 = 32-bit offsets (0 and 2: blocks as registers allow); 3 = both kernels staged
         bool patch;  // two-stage: the runs' tile patches (else rows of tiles)
     };
     std::vector<Cand> cands;
+    // the shape the batch was made with: fused here, two-stage below (without
+    // LDS its 64 x 2 tiles of short chunks are within 3 % of 64 x 4)
+    if (!b->split)
+        cands.push_back({false, true, b->l.tile_y, b->l.unroll, swept(b, b->l.tile_y, b->l.unroll) ? 0 : b->nchunk[0],
+                         1, 0, true});
     // two-stage, one block per tile, chunk lengths about the default's
-    for (int kc : {b->kc_split * 2 / 3, b->kc_split, b->kc_split * 3 / 2})
-        for (bool pt : {true, false}) cands.push_back({true, false, 4, 1, std::max(4, kc), 1, b->o32 ? 2 : 0, pt});
+    {
+        const int d = plain_levels(b);
+        for (int kc : {d, d * 2 / 3, d * 3 / 2})
+            for (bool pt : {true, false}) cands.push_back({true, false, 4, 1, std::max(4, kc), 1, b->o32 ? 2 : 0, pt});
+    }
     {
         Launch sl = b->l;
         sl.unroll = sl.tile_xw = 1;
         sl.bpc_v = sl.bpc_s = 0;
+        const int d = staged_levels(b);
         if (staged_shape(sl))
-            for (int kc : {b->kc_split * 2 / 3, b->kc_split, b->kc_split * 3 / 2})
+            for (int kc : {d, d * 2 / 3, d * 3 / 2})
                 cands.push_back({true, false, STAGED_TY, 1, std::max(4, kc), 1, 3, true});
     }
     for (bool ps : {true, false}) {
@@ -541,7 +559,8 @@ extern "C" int awp_batch_tune(awp_batch *b, int reps)
         const int tp[8][2] = {{11, 3}, {11, 0}, {8, 0}, {7, 0}, {7, 1}, {7, 2}, {4, 0}, {4, 2}};
         if (b->can_fuse)
             for (const auto &v : tp)
-                for (int nc : {2, 4}) cands.push_back({false, ps, v[0], v[1], nc, 1, 0, true});
+                for (int nc : {0, 2, 4})
+                    if (nc || swept(b, v[0], v[1])) cands.push_back({false, ps, v[0], v[1], nc, 1, 0, true});
     }
     const int spw0 = b->l.spw, sph0 = b->l.sph;
     auto apply_form = [b, spw0, sph0](int sf, bool patch) {
@@ -552,19 +571,24 @@ extern "C" int awp_batch_tune(awp_batch *b, int reps)
         b->l.sph = patch ? sph0 : 0;
         set_block_caps(b->l, b->device);
     };
-    // times the step kernels of candidate cd over n launches after one
-    // warm-up (ms in *out)
-    auto time_cand = [&](const Cand &cd, int n, double *out) -> int {
+    auto take = [&](const Cand &cd) {
         b->split = cd.split;
         b->persist = cd.persist;
         apply_form(cd.sform, cd.patch);
         b->l.tile_y = cd.ty;
         b->l.tile_xw = cd.xw;
         b->l.unroll = cd.pf;
-        if (cd.split)
+        if (cd.split) {
             b->kc_split = cd.nchunk;
-        else
-            std::fill(b->nchunk.begin(), b->nchunk.end(), cd.nchunk);
+        } else {
+            fused_patch(b->l, b->mixed);
+            std::fill(b->nchunk.begin(), b->nchunk.end(), cd.nchunk ? cd.nchunk : sweep_chunks(b));
+        }
+    };
+    // times the step kernels of candidate cd over n launches after one
+    // warm-up (ms in *out)
+    auto time_cand = [&](const Cand &cd, int n, double *out) -> int {
+        take(cd);
         int rc = upload_tables(b);
         if (rc) return rc;
         set_grids(b);
@@ -588,7 +612,7 @@ extern "C" int awp_batch_tune(awp_batch *b, int reps)
         if (log)
             fprintf(stderr, "awp_batch_tune %s: %s %s ty %d xw %d pf/unroll %d chunks %d form %d patch %d: %.3f ms\n",
                     pass, cd.split ? "two-stage" : "fused", cd.persist ? "persistent" : "per-tile", cd.ty, cd.xw,
-                    cd.pf, cd.nchunk, cd.sform, cd.patch ? 1 : 0, ms);
+                    cd.pf, cd.split ? b->kc_split : b->nchunk[0], cd.sform, cd.patch ? 1 : 0, ms);
     };
     std::vector<std::pair<double, size_t>> first;
     for (size_t n = 0; n < cands.size(); ++n) {
@@ -611,16 +635,7 @@ extern "C" int awp_batch_tune(awp_batch *b, int reps)
             pick = cands[first[q].second];
         }
     }
-    b->split = pick.split;
-    b->persist = pick.persist;
-    apply_form(pick.sform, pick.patch);
-    b->l.tile_y = pick.ty;
-    b->l.tile_xw = pick.xw;
-    b->l.unroll = pick.pf;
-    if (pick.split)
-        b->kc_split = pick.nchunk;
-    else
-        std::fill(b->nchunk.begin(), b->nchunk.end(), pick.nchunk);
+    take(pick);
     set_grids(b);
     drop_graph(b);
     // the trial steps changed the runs' state: start them again

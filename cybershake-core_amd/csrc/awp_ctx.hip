@@ -170,6 +170,23 @@ static void set_chunks(Launch &l, const Geo &g, int nchunk, bool fused)
     l.nchunk = (g.nz + l.kc - 1) / l.kc;
 }
 
+// tile patches of the fused step (AWP_PATCH=<w>x<h> overrides): FP32 64 x 11
+// 2 x 2 (1500x1000x300: 14.64 ms per step against 14.72 for 4 x 4, 14.88 for
+// 8 x 2, 15.06 for rows and 15.14 for 3 x 3), else 4 x 4 (64 x 8, 4 z chunks:
+// 17.21 against 17.62 for 2 x 16 and 17.75 for 3 x 8)
+void fused_patch(Launch &l, bool mixed)
+{
+    l.pw = l.ph = l.tile_y == 11 && !mixed ? 2 : 4;
+    const char *pe = getenv("AWP_PATCH");
+    if (pe) {
+        int w = 0, h = 0;
+        if (sscanf(pe, "%dx%d", &w, &h) == 2 && w >= 1 && h >= 1 && w * h <= 4096) {
+            l.pw = w;
+            l.ph = h;
+        }
+    }
+}
+
 Launch choose_launch(const Geo &g, bool fused, bool mixed, int device)
 {
     Launch l;
@@ -199,11 +216,7 @@ Launch choose_launch(const Geo &g, bool fused, bool mixed, int device)
         l.tile_y = atoi(ty);
     if (fused && l.tile_y != 4 && l.tile_y != 7 && l.tile_y != 11) l.tile_y = 8;
     if (!fused && (l.tile_y == 7 || l.tile_y == 11)) l.tile_y = 8;
-    // tile patches of the fused step (AWP_PATCH=<w>x<h> overrides): FP32 64 x
-    // 11 2 x 2 (1500x1000x300: 14.64 ms per step against 14.72 for 4 x 4, 14.88
-    // for 8 x 2, 15.06 for rows and 15.14 for 3 x 3), else 4 x 4 (64 x 8, 4 z
-    // chunks: 17.21 against 17.62 for 2 x 16 and 17.75 for 3 x 8)
-    l.pw = l.ph = fused && l.tile_y == 11 && !mixed ? 2 : 4;
+    fused_patch(l, mixed);
     // tile claim (AWP_CLAIM=0 never, 1 when the launch has at least four
     // tiles per persistent block, 2 always; AWP_XROT=0..7 rotates the XCD
     // ranges): persistent blocks that claim tiles per XCD.  The default of
@@ -218,14 +231,6 @@ Launch choose_launch(const Geo &g, bool fused, bool mixed, int device)
     if (ce && (!strcmp(ce, "0") || !strcmp(ce, "1") || !strcmp(ce, "2"))) l.claim = ce[0] - '0';
     const char *xr = getenv("AWP_XROT");
     if (xr) l.xrot = atoi(xr) & 7;
-    const char *pe = getenv("AWP_PATCH");
-    if (pe) {
-        int w = 0, h = 0;
-        if (sscanf(pe, "%dx%d", &w, &h) == 2 && w >= 1 && h >= 1 && w * h <= 4096) {
-            l.pw = w;
-            l.ph = h;
-        }
-    }
     l.o32 = use_o32(g);
     // AWP_CACHED=0..3 overrides the two-stage kernels' cache mode
     l.cached = fused ? 0 : cache_mode(g.nvol, mixed);

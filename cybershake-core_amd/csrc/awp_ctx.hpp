@@ -112,6 +112,8 @@ struct awp_ctx {
 
 // the default launch shape of a run of these sizes by either scheme
 Launch choose_launch(const Geo &g, bool fused, bool mixed, int device);
+// the fused step's tile patches for l's tiles
+void fused_patch(Launch &l, bool mixed);
 
 inline int fail(awp_ctx *ctx, int code, const char *fmt, ...)
 {

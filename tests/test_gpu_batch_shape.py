@@ -77,3 +77,37 @@ def test_batch_scheme_by_all_runs_sizes(tmp_path, monkeypatch):
             assert np.array_equal(r.field(f), ref.field(f)), f
         r.close()
         ref.close()
+
+
+@pytest.mark.parametrize("scheme", ["fused", "split"])
+def test_tuner_tries_the_shape_it_was_given(scheme, tmp_path, monkeypatch, capfd):
+    """Tuning a batch that is on its default shape times that shape too (the
+    staged two-stage tiles, the FP32 fused step with its z chunks)."""
+    sizes = [(70, 34, 56), (48, 40, 32), (130, 25, 24)]
+    refs = _runs(tmp_path, sizes)
+    monkeypatch.setenv("AWP_STAGED", "1")
+    runs = _runs(tmp_path, sizes)
+    monkeypatch.setenv("AWP_BATCH_SCHEME", scheme)
+    monkeypatch.setenv("AWP_TUNE_LOG", "1")
+    with awpsgt.Batch(runs) as b:
+        ty, pf, chunks = b.launch()
+        assert (ty, pf) == ((11, 3) if scheme == "fused" else (8, 1))
+        capfd.readouterr()
+        b.tune(1)
+        tried = [ln.split() for ln in capfd.readouterr().err.splitlines() if ln.startswith("awp_batch_tune first")]
+        assert len(tried) > 20
+        if scheme == "fused":
+            # scheme, grid, "ty", rows, "xw", waves, "pf/unroll", depth, "chunks", chunks
+            assert ["fused", "persistent", "ty", "11", "xw", "1", "pf/unroll", "3", "chunks", str(chunks)] in \
+                [t[2:12] for t in tried]
+        else:
+            # staged: form 3; a run's chunks from the levels a chunk, at least 8 each
+            kcs = [int(t[11]) for t in tried if t[2] == "two-stage" and t[13] == "3"]
+            assert any(min((56 + kc // 2) // kc, 56 // 8) == chunks for kc in kcs)
+        b.step(runs[0].p.nt)
+    for r, ref in zip(runs, refs):
+        ref.step(ref.p.nt)
+        ref.synchronize()
+        _equal(ref, r)
+        r.close()
+        ref.close()
