@@ -8,14 +8,15 @@
 // up to four waves and at up to five x offsets, and the vector cache stalls on
 // every access to a line that is still on its way -- 58 % (velocity) and 63 %
 // (stress) of their cycles at 1500x1000x300 (TCP_PENDING_STALL_CYCLES).  Here
-// a wave loads 11 (13) lines a level and 1.8 (2.5) more for the surroundings,
-// instead of 30 (45).  us per step, velocity / stress, without -> with:
-// 1500x1000x300 FP32 5200 / 11980 -> 4790 / 11490, mixed 5016 / 9130 -> 4604 /
-// 8727; 517x389x149 FP32 370 / 842 -> 335 / 788, mixed 356 / 658 -> 325 / 615.
-// That is 5.0 TB/s for the stress kernel, the rate of bare streams in its mix
-// of reads and writes; 64 x 8 tiles, as 64 x 4 spill scalar registers (the
-// halo loads of five items a wave) and 64 x 16 wait at longer barriers (16.29
-// / 16.38 / 16.63 ms per step with 8 / 4 / 16 rows).
+// a wave has 10 (stress: 19 FP32, 17 mixed) loads a level of its own point's
+// values and 1.8 (2.5, 2.0) for the surroundings, instead of 31 (49, 41).
+// us per step, velocity / stress, without -> with: 1500x1000x300 FP32 5200 /
+// 11980 -> 4790 / 11490, mixed 5016 / 9130 -> 4604 / 8727; 517x389x149 FP32
+// 370 / 842 -> 335 / 788, mixed 356 / 658 -> 325 / 615.  That is 5.0 TB/s for
+// the stress kernel, the rate of bare streams in its mix of reads and writes;
+// 64 x 8 tiles, as 64 x 4 spill scalar registers (the halo loads of five items
+// a wave) and 64 x 16 wait at longer barriers (16.29 / 16.38 / 16.63 ms per
+// step with 8 / 4 / 16 rows).
 // Statements and their order are those of velocity_tile_b / stress_tile_b.
 #pragma once
 #include "awp_kernels.hpp"
@@ -359,7 +360,10 @@ __device__ __forceinline__ void stress_tile_s(const Geo &g, const State &s0, con
     float hv[NS];
 #pragma unroll
     for (int t = 0; t < NS; ++t) hv[t] = hl[t].kind ? load_halo(hl[t]) : 0.0f;
-    __syncthreads();   // the planes of the block's tile before
+    // (not needed for the LDS, which nothing has touched yet: it lines up the
+    // waves after their start-up loads, mixed 400x300x150 382 us against 384
+    // without it, FP32 and larger grids the same within 0.1 %)
+    __syncthreads();
     int m0 = kb % 3, mp = (kb + 2) % 3;   // media slots of levels k and k-1
     float mb0 = 0.f, lb0 = 0.f;
     if constexpr (P::mixed) { mb0 = s.mbar[mbar_idx(g, 1, kb - 1)]; lb0 = s.mbar[mbar_idx(g, 2, kb - 1)]; }

@@ -1,7 +1,8 @@
 """Two levels per barrier of the mixed fused step on 64 x 11 tiles where the
 level pair meets the free surface: where the pair (nz, nz + 1) falls in one
-group (nz - kb even, kb the chunk's first level), the velocity images at nz + 1 wait for level nz behind a barrier of their
-own.  (FP32 takes another body on these tiles.)"""
+group (nz - kb even, kb the chunk's first level), the velocity images at
+nz + 1 wait for level nz behind a barrier of their own.  (FP32 takes another
+body on these tiles.)"""
 import numpy as np
 import pytest
 
