@@ -190,14 +190,17 @@ void fused_patch(Launch &l, bool mixed)
 Launch choose_launch(const Geo &g, bool fused, bool mixed, int device)
 {
     Launch l;
-    // two-stage: 64 x 4 tiles, 64 x 2 where the chunks are short (split_kc).
-    // Low tiles share no less in the caches than tall ones (the L2 serves
-    // both) and small blocks fill the wave slots evenly: one block per tile,
-    // ms per step with 2 / 4 / 8 rows, FP32 and mixed: 131x97x53 (4 levels)
-    // 0.060 / 0.062 / 0.066 and 0.059 / 0.061 / 0.064; 400x300x150 (17) 0.749
-    // / 0.749 / 0.771 and 0.636 / 0.639 / 0.659; 1410x88x77 (13) 0.427 /
-    // 0.404 / 0.394; 800x600x200 (25) 3.60 / 3.62 / 3.65 and 2.99 / 2.99 /
-    // 3.02; 1500x1000x300 17.08 / 17.17 / 17.25 and 14.21 / 14.20 / 14.28
+    // two-stage without LDS: 64 x 4 tiles, 64 x 2 where the chunks are short
+    // (split_kc).  Low tiles share no less in the caches than tall ones (the
+    // L2 serves both) and small blocks fill the wave slots evenly: one block
+    // per tile, us per step with 1 / 2 / 4 / 8 rows, FP32 and mixed: 48x40x32 (4
+    // levels) 12.9 / 13.0 / 14.4 / 18.0 and 17.9 / 17.9 / 18.7 / 22.0;
+    // 131x97x53 (4) 32.3 / 33.0 / 34.8 / 34.5 and 35.8 / 35.8 / 36.9 / 37.2;
+    // 400x300x150 (17) 709 / 705 / 706 / 730 and 594 / 592 / 596 / 622;
+    // 1410x88x77 (13) 385 / 382 / 374 / 365 and 324 / 323 / 322 / 322;
+    // 800x600x200 (25) 3565 / 3569 / 3577 / 3628 and 2949 / 2941 / 2943 / 2991;
+    // 1500x1000x300 17160 / 17060 / 17170 / 17210 and 14240 / 14150 / 14140 /
+    // 14260 (the last four are staged by default)
     l.tile_y = split_kc(row_segments(g), g.nz) > 8 ? 4 : 2;
     l.tile_xw = 1;
     l.unroll = 1;

@@ -1484,8 +1484,8 @@ void set_staged(Launch &l)
 
 // The staged form unless the run fits the memory-side cache whole, or (mixed)
 // all of it but r1..r6: there a step is bound by the chain of a wave's
-// levels, which the barrier of each lengthens.  us per step without / with,
-// FP32: 48x40x32 27 / 32, 150x150x90 79 / 89, 180x160x90 (mode 2) 111 / 102,
+// levels, which the barrier of each lengthens.  us per step (timing events of
+// some 13 us included) without / with, FP32: 48x40x32 27 / 32, 150x150x90 79 / 89, 180x160x90 (mode 2) 111 / 102,
 // 203x187x101 168 / 163, 240x220x80 171 / 152, 260x220x100 267 / 237,
 // 517x389x149 1219 / 1132, 800x600x200 3595 / 3430, 1500x1000x300 17194 /
 // 16292; mixed: 48x40x32 32 / 38, 150x150x90 78 / 97, 180x160x90 89 / 100,

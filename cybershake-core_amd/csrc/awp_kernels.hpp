@@ -419,19 +419,22 @@ struct Cursor32 {
 constexpr int STAGED_TY = 8;
 
 // z chunk length of the two-stage kernels without LDS for `rows` row segments of 64
-// points a level and nz levels.  A wave marches its chunk level by level, 2.9
-// us each on an idle GPU (load, compute, store), so a grid that cannot fill
-// the GPU's 4096 wave slots (4 per SIMD) is bound by that chain and takes
-// short chunks: about three waves per slot, 4 to 17 levels each (below 4 the
-// z queues' start-up loads cost more than the shorter chain saves).  From
-// twelve waves per slot on the chain is hidden and 25-level chunks, with
-// fewer start-up loads, win.  Milliseconds per step, 64 x 2 tiles, one block
-// per tile, FP32 / mixed: 48x40x32 with 4 / 12 levels 0.032 / 0.044 and
-// 0.037 / 0.049; 131x97x53 with 4 / 25 levels 0.060 / 0.092 and 0.059 /
-// 0.124; 300x250x80 with 8 / 25 0.261 / 0.275 and 0.231 / 0.257; 400x300x150
-// with 17 / 25 0.749 / 0.765 and 0.636 / 0.668; 800x600x200 with 17 / 25 3.71
-// / 3.60 and 3.07 / 2.99; 1500x1000x300 with 12 / 17 / 25 / 50 17.25 / 17.23 /
-// 17.08 / 17.39 and 14.37 / 14.32 / 14.21 / 14.32.
+// points a level and nz levels.  A wave marches its chunk level by level: on
+// an idle GPU 1.8 us a level, both kernels together (48x40x32: 13.3 us a step
+// in chunks of 4 levels, 63.4 in one of 32), so a grid that cannot fill the
+// GPU's 4096 wave slots (4 per SIMD) is bound by that chain and takes short
+// chunks: about three waves per slot, 4 to 17 levels each.  From twelve waves
+// per slot on the chain is hidden and 25-level chunks, with fewer start-up
+// loads, win.  Microseconds per step, one block per tile, FP32 and mixed, in
+// chunks of the levels given: 48x40x32 4 / 8 / 12 13.4 / 20.7 / 25.7 and 17.9 /
+// 29.2 / 37.3; 131x97x53 4 / 8 / 25 33.0 / 36.0 / 47.4 and 35.9 / 40.4 / 69.6;
+// 200x200x100 4 / 6 / 8 / 13 168 / 166 / 167 / 175 and 142 / 143 / 144 / 152;
+// 300x250x80 4 / 8 / 13 237 / 233 / 242 and 206 / 206 / 216; 400x300x150 8 / 13 /
+// 17 / 25 743 / 716 / 706 / 719 and 609 / 605 / 596 / 616; 800x600x200 12 / 17 /
+// 25 / 50 3738 / 3690 / 3577 / 3690 and 3064 / 3033 / 2943 / 3034;
+// 1500x1000x300 12 / 17 / 25 / 50 17190 / 17270 / 17170 / 17260 and 14300 /
+// 14290 / 14140 / 14260 (the last four, and FP32 200x200x100, are staged by
+// default).
 static inline int split_kc(long long rows, int nz)
 {
     const long long waves = rows * nz;   // row segments over the whole volume

@@ -4,16 +4,18 @@
 // (Halo), bring the rows and columns around the tile.  The loads of the next
 // level are issued before the current one's arithmetic, one barrier a level.
 //
-// What the forms without LDS lose: each row of a stencil array is loaded by
-// up to four waves and at up to five x offsets, and the vector cache stalls on
-// every access to a line that is still on its way -- 58 % (velocity) and 63 %
-// (stress) of their cycles at 1500x1000x300 (TCP_PENDING_STALL_CYCLES).  Here
-// a wave has 10 (stress: 19 FP32, 17 mixed) loads a level of its own point's
-// values and 1.8 (2.5, 2.0) for the surroundings, instead of 31 (49, 41).
+// In the forms without LDS each row of a stencil array is loaded by up to four
+// waves and at up to five x offsets: 31 loads a point and level in the velocity
+// kernel, 49 (mixed 41) in the stress kernel.  Here a wave has 10 (stress: 19
+// FP32, 17 mixed) for its own points and 1.8 (2.5, 2.0) for the surroundings;
+// at 1500x1000x300 FP32 170M and 287M wave loads a launch become 95M and 166M.
 // us per step, velocity / stress, without -> with: 1500x1000x300 FP32 5200 /
 // 11980 -> 4790 / 11490, mixed 5016 / 9130 -> 4604 / 8727; 517x389x149 FP32
 // 370 / 842 -> 335 / 788, mixed 356 / 658 -> 325 / 615.  That is 5.0 TB/s for
-// the stress kernel, the rate of bare streams in its mix of reads and writes;
+// the stress kernel, the rate of bare streams in its mix of reads and writes.
+// The vector cache waits for lines on their way in both forms, for fewer loads
+// a larger part of the time (TCP_PENDING_STALL_CYCLES, velocity / stress: 59 /
+// 63 % of the cycles without, 79 / 81 % with): the time is the memory's.
 // 64 x 8 tiles, as 64 x 4 spill scalar registers (the halo loads of five items
 // a wave) and 64 x 16 wait at longer barriers (16.29 / 16.38 / 16.63 ms per
 // step with 8 / 4 / 16 rows).

@@ -12,14 +12,15 @@
 // and whose z neighbours are the thread's own.  Statements and their order
 // are those of step_tile.
 //
-// What bounds step_tile is the vector cache: each row of a stencil array is
-// loaded by up to four waves at up to five offsets, 52 loads a point, and 67 %
-// of its cycles stall on lines on their way; neither deeper prefetch nor less
-// traffic from memory (regions of tiles that fit the L2s) changed its time.
-// Here a row takes 20 loads and an item wave 5 more.  A CU holds one block of
-// 16 waves in step with each other, so what counts next is that a level has
-// one wait: all loads of the next level are issued after the barrier, and
-// waited for together before the level's stores, which no wait then includes
+// step_tile loads each row of a stencil array by up to four waves at up to five
+// offsets, 52 loads a point, 389M wave loads a launch at 1500x1000x300; neither
+// deeper prefetch nor less traffic from memory (regions of tiles that fit the
+// L2s) changed its time.  Here a row takes 20 loads and an item wave 5 more,
+// 223M a launch.  (The vector cache waits for lines on their way 67 % of the
+// cycles there, 71 % here.)  A CU holds one block of 16 waves in step with each
+// other, so what counts next is that a level has one wait: all loads of the
+// next level are issued after the barrier, and waited for together before the
+// level's stores, which no wait then includes
 // (waiting at the top of the next level, behind the stores: 20.2 ms per step;
 // stores of the stresses alone behind the wait: 15.1).  FP32, ms per step
 // before -> after, against two-stage staged: 517x389x149 1.29 -> 1.10 (1.13),

@@ -173,12 +173,16 @@ int awp_sgt_compare(const char *ref_path, const char *test_path, long long npts,
 /* Create a context on HIP device `device` (allocates every device buffer;
  * replaces the host's cudaMalloc block, pmcl3d.c:537-823, and
  * SetDeviceConstValue, kernel...cu:24).  Two time-step schemes give the same
- * bits: the two-stage step (velocity kernel, free-surface images, stress
- * kernel, in place) and the one-sweep fused step, which reads one wavefield
- * buffer and writes a second one (36 more bytes per grid point).  FP32 runs
- * take the fused step, mixed-storage runs the two-stage one; AWP_SCHEME=split
- * or AWP_SCHEME=fused in the environment overrides (grids whose arrays reach
- * 4 GiB always take the two-stage step). */
+ * bits: the two-stage step (velocity kernel, then the stress kernel, which
+ * makes the free-surface images too; in place) and the one-sweep fused step,
+ * which reads one wavefield buffer and writes a second one (36 more bytes per
+ * grid point).  FP32 runs hold both buffers and take the fused step from 25M
+ * points on, the two-stage one below, where the second buffer (allocated,
+ * zeroed by awp_init and checkpointed all the same) serves awp_tune,
+ * awp_set_scheme and fused batches only; mixed-storage runs hold one buffer
+ * and take the two-stage step.  AWP_SCHEME=split (one buffer) or
+ * AWP_SCHEME=fused in the environment overrides; grids whose planes exceed
+ * some 40M points always take the two-stage step. */
 int awp_create(awp_ctx **out, const awp_in3d *p, int device, int storage,
                char *err, size_t errlen);
 int awp_destroy(awp_ctx *ctx);
@@ -212,12 +216,12 @@ int awp_init(awp_ctx *ctx);
 
 /* Time-step scheme of a run; every scheme and launch shape gives the same
  * bits.  awp_tune times `reps` steps (default 3) of each candidate -- the
- * two-stage step (on grids of few tiles also with 64x4 tiles and shorter z
- * chunks) and, in a run that holds the second wavefield buffer, the fused
- * step on several tile, z-chunk and tile-patch shapes --, times the three
- * fastest again over twice the steps, keeps the fastest and starts the run
- * again (awp_init): call it on an initialised run before its first step.  awp_set_scheme(ctx, 1 / 0) switches to the fused /
- * two-stage step with its default launch shape at any point between steps
+ * two-stage step (its default, the staged form with other z chunks, and where
+ * that is not the default other tiles too) and, in a run that holds the second
+ * wavefield buffer, the fused step on several z-chunk and tile-patch shapes --,
+ * times the three fastest again over twice the steps, keeps the fastest and
+ * starts the run again (awp_init): call it on an initialised run before its
+ * first step.  awp_set_scheme(ctx, 1 / 0) switches to the fused / two-stage step with its default launch shape at any point between steps
  * (the fused step needs the second buffer).  awp_get_scheme reports the step
  * in use (1 fused, 0 two-stage), its tile rows and its z chunks; any pointer
  * may be NULL.  No counterpart in the reference, which has one kernel
@@ -238,7 +242,11 @@ int awp_progress(const awp_ctx *ctx, int *step, int *nsamples);
 
 /* SGT samples so far, [npts][6][nsamp_max] float32 with nsamp_max =
  * nt / NTISKP_SGT; slots of points the rule drops and samples not yet taken
- * are -1.  (Strains exx eyy ezz exy exz eyz, pmcl3d.f:1546-1557.) */
+ * are -1.  (Strains exx eyy ezz exy exz eyz, pmcl3d.f:1546-1557.)  Once the
+ * output read and written from a run adds up to 64 MB, the run keeps 32 MB of
+ * pinned host memory for it until awp_destroy (without, transfers go through
+ * pageable memory).  This call and the file writers may run in several
+ * threads at once on a run that is not stepping. */
 int awp_get_sgt(awp_ctx *ctx, float *host, size_t count);
 
 /* The job-value trace the reference's master rank writes to the CHKJ file
@@ -261,7 +269,8 @@ int awp_write_sgt_file(awp_ctx *ctx, const char *path);
  * with XX <- YY, YY <- XX, XZ <- -YZ, YZ <- -XZ, every value first times -2
  * when zsource != 0 (the Z-force component), complete records of the raw
  * file only, its holes as zeros.  Replaces awp_write_sgt_file + reformat_awp
- * (reformat_awp_mpi.c:91-122) in a CyberShake SGT workflow. */
+ * (reformat_awp_mpi.c:91-122) in a CyberShake SGT workflow.  Written from
+ * start to end, so `path` may be a pipe (as in awp_write_sgt_file_fp16). */
 int awp_write_sgt_file_rwg(awp_ctx *ctx, const char *path, int zsource);
 
 /* Write the SGT in the compact FP16 format (no counterpart in the
@@ -371,20 +380,22 @@ int awp_write_sgt_head(const awp_head_params *hp, char *err, size_t errlen);
 
 /* ---- batches ------------------------------------------------------------
  * Several initialised runs (same device and storage mode) advanced
- * together: each stage of a time step is one persistent launch over the
- * tiles of every run (two-stage scheme: velocity, free-surface images,
- * stress; fused scheme: the one-sweep kernel), then one launch for every
- * run's source and SGT sample, replayed from a HIP graph.  The fused scheme
- * is used when every run holds two wavefield buffers and steps fused (the
- * FP32 default, or AWP_SCHEME=fused), else the two-stage one.  Each run keeps its own
- * outputs (awp_get_sgt, awp_write_sgt_file).  The reference runs one SGT
+ * together: each stage of a time step is one launch over the tiles of every
+ * run (two-stage scheme: velocity, stress; fused scheme: the one-sweep
+ * kernel), then the launches for every run's source and SGT sample, replayed
+ * from a HIP graph.  The fused scheme is used when every run holds two
+ * wavefield buffers and either steps fused, or steps two-stage by its size
+ * alone (not by awp_set_scheme or awp_tune) while the runs have 25M points
+ * together; else the two-stage one.  Each run keeps its own outputs
+ * (awp_get_sgt, awp_write_sgt_file).  The reference runs one SGT
  * component per MPI job (AWP-ODC-SGT/utils/awp_odc_wrapper.sh:14); these
  * entry points have no counterpart in it. */
 typedef struct awp_batch awp_batch;
 int awp_batch_create(awp_batch **out, awp_ctx *const *runs, int nruns, char *err, size_t errlen);
-/* Times the batch's step kernels for each scheme (fused only when the runs
- * hold two buffers) / tile height / prefetch depth or z unroll / z chunking
- * / persistent or one-block-per-tile grid candidate (reps launches each),
+/* Times the batch's step kernels in the shape it was made with and for each
+ * scheme (fused only when the runs hold two buffers) / tile height / prefetch
+ * depth or z unroll / z chunking / persistent or one-block-per-tile grid
+ * candidate (reps launches each),
  * times the three fastest again over twice the launches and keeps the
  * fastest.  Needs runs that have not stepped; re-initialises them
  * (awp_init) afterwards. */
